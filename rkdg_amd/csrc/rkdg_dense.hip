@@ -11,72 +11,156 @@
 // (nodal flux, GetFlux fe_evolution.cpp:219-245) and K_r(j,k) the exact integral
 // of phi_k d_r phi_j (triangles; DomainIntegrator with intorder 2p is exact) or
 // the collocated w_k d_r phi_j(x_k) with adj(J) taken at node k (Q_p on
-// Gauss-Legendre nodes). Faces: per-face trace tables Phi_f[q][k]; the
-// neighbour's trace is evaluated at the mirrored point of its own face. Mass:
-// M^-1 = Mhat^-1 / det J (affine triangles) or a per-element dense inverse
-// (bilinear quads).
+// Gauss-Legendre nodes). Faces: the neighbour's trace is evaluated at the
+// mirrored point of its own face. Mass: M^-1 = Mhat^-1 / det J (affine
+// triangles); on a bilinear quadrilateral det J is linear in each coordinate, so
+// the p+1 point Gauss-Legendre rule integrates phi_i phi_j det J exactly and the
+// mass matrix is diagonal, w_j det J(x_j).
 #include "rkdg_dense.hpp"
 
 namespace rkdg {
 
+// Right-hand side. One lane per face point: T = NF * NQ lanes per element and
+// 64 / T elements per wavefront (P2 triangles: 7 elements fill 63 lanes, where a
+// power-of-two team of 16 lanes left 28 of 64 idle in the Riemann solves, the
+// longest phase). The neighbours' states are read one (face, variable) row per
+// lane, contiguous and once, instead of whole by each face point; quadrilaterals
+// interpolate a row to the face points in registers (sum-factorised, tables read
+// once per lane), triangles stage it in LDS. Geometry is formed from the edge
+// normals alone (adj(J) and det J are polynomials in the edge vectors), so an
+// element reads 2 NF doubles of its record, and the inverse mass is folded into
+// the volume and lift tables (triangles) or diagonal (quadrilaterals).
+//
+// Bound by FP64 issue and latency at 3 waves per SIMD. Limited steps, before
+// (power-of-two teams, every point reading the whole neighbour, dense inverse
+// mass and a full geometry record per element) and now: 27,467 bilinear Q2
+// quadrilaterals, two stages, HLLC 229 -> 108 us; 120,540 P2 triangles, three
+// stages, HLLC 488 -> 268 us; 472,000 Q1 quadrilaterals in 64 instances, eight
+// steps of three stages, HLL 12.9 -> 7.9 ms.
+template <int GEOM, int P>
+struct RC : DC<GEOM, P> {
+  using D = DC<GEOM, P>;
+  static constexpr int N = P + 1;
+  static constexpr int T = D::NPT;
+  static constexpr int EPB = D::BLOCK / T;
+  static constexpr int ROWS = D::NF * D::NEQ;       // neighbour rows (face, variable)
+  static constexpr int RP = (ROWS + T - 1) / T;     // rows per lane
+};
+
+// Keeps the scheduler from moving loads across this point: the unrolled
+// contractions would otherwise have every LDS read in flight at once (255 VGPRs
+// and spills on P2 triangles).
+__device__ __forceinline__ void hold() { __builtin_amdgcn_sched_barrier(0); }
+
+// Keeps a contraction in its basic block: the compiler otherwise sinks the
+// arithmetic below the branches of the epilogue and leaves its LDS reads, all
+// of them live, above (spills).
+template <int n>
+__device__ __forceinline__ void pin(double* y) {
+#pragma unroll
+  for (int v = 0; v < n; v++) asm volatile("" : "+v"(y[v]));
+}
+
 // one work block (EPB elements, one wavefront) of the right-hand side
 template <int GEOM, int P, int RS, bool BC>
 __device__ __forceinline__ void dense_rhs_block(const RhsArgs& A, const SchemeParams& g, int64_t vb,
-                                                DenseTab<GEOM, P>& tb) {
-  using C = DC<GEOM, P>;
-  constexpr int ND = C::ND, NEQ = C::NEQ, NF = C::NF, NQ = C::NQ, NPT = C::NPT;
-  constexpr int T = C::T, EPB = C::EPB, BLOCK = C::BLOCK, GS = C::GSIZE;
+                                                DenseRhsTab<GEOM, P>& tb) {
+  using C = RC<GEOM, P>;
+  constexpr int N = C::N, ND = C::ND, NEQ = C::NEQ, NF = C::NF, NQ = C::NQ, NPT = C::NPT;
+  constexpr int T = C::T, EPB = C::EPB, BLOCK = C::BLOCK, RP = C::RP;
   constexpr bool TRI = C::TRI;
+  // traces: quadrilaterals hold the values at the face points, own and the
+  // neighbour's (index along the axis), triangles the neighbours' node values
+  constexpr int TR = TRI ? NF * NEQ * ND : 2 * NF * NQ * NEQ;
 
-  __shared__ double s_u[EPB][NEQ][ND];
-  __shared__ double s_g[EPB][2][NEQ][ND];     // contravariant nodal fluxes, then z
-  __shared__ double s_f[EPB][NPT][NEQ];       // weighted face fluxes
-  __shared__ double s_geo[EPB][GS];
+  __shared__ __attribute__((aligned(16))) double s_u[EPB][NEQ][ND];
+  __shared__ __attribute__((aligned(16))) double s_g[EPB][2][NEQ][ND];  // contravariant nodal fluxes, then the means
+  __shared__ __attribute__((aligned(16))) double s_t[EPB][TR];
+  __shared__ __attribute__((aligned(16))) double s_f[EPB][NPT][NEQ];    // weighted face fluxes
+  __shared__ double s_nrm[EPB][2 * NF];
   __shared__ int s_nb[EPB][NF], s_code[EPB][NF];
 
-  const int tid = threadIdx.x;
-  const int team = tid / T, lane = tid % T;
+  // opaque to the compiler, so that the LDS addresses formed from it are not
+  // kept over the persistent loop (they held 160 registers and spilled)
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  const int team = tid / T, lane = tid - team * T;
   const int64_t NE = A.NE;
   const int64_t NDOFS = NE * ND;
   const int64_t e0 = vb * EPB;
   const int64_t e = e0 + team;
-  const int ins = (A.inst && e < NE) ? A.inst[e] : 0;
-  const bool active = e < NE && (!A.active || A.active[ins]);
+  const bool in = team < EPB && e < NE;
+  const int ins = (A.inst && in) ? A.inst[e] : 0;
+  const bool active = in && (!A.active || A.active[ins]);
 
-  // every load of the block's setup is issued before the first LDS store
-  static_assert(NF <= T, "one lane per face");
+  // every load of the block's setup is issued before the first LDS store; the
+  // neighbours' rows, which need the connectivity, follow in one more round trip
+  static_assert(2 * NF <= T && ND <= T, "one lane per normal component and node");
   StateRegs<EPB, NEQ, ND, BLOCK> str;
   str.load(A.x, NDOFS, e0, NE, tid);
-  constexpr int GSP = (GS + T - 1) / T;
-  double gv[GSP];
-#pragma unroll
-  for (int p = 0; p < GSP; p++) gv[p] = (active && lane + p * T < GS) ? A.geo[(int64_t)(lane + p * T) * NE + e] : 0.0;
+  const double nv = (active && lane < 2 * NF) ? A.geo[(int64_t)(C::G_NRM + lane) * NE + e] : 0.0;
   const bool face_lane = active && lane < NF;
   const int nb0 = face_lane ? A.nbr[lane * NE + e] : -1;
   const int cd0 = face_lane ? A.fcode[lane * NE + e] : 0;
+  int rnb[RP];
+#pragma unroll
+  for (int p = 0; p < RP; p++) {
+    const int it = lane + p * T;
+    rnb[p] = (active && it < C::ROWS) ? A.nbr[(it / NEQ) * NE + e] : -1;
+  }
+  double row[RP][ND];
+#pragma unroll
+  for (int p = 0; p < RP; p++) {
+    if (rnb[p] >= 0) {
+      const double* xn = A.x + (int64_t)((lane + p * T) % NEQ) * NDOFS + (int64_t)rnb[p] * ND;
+#pragma unroll
+      for (int k = 0; k < ND; k++) row[p][k] = xn[k];
+    }
+  }
   str.store(s_u, tid);
   if (face_lane) {
     s_nb[team][lane] = nb0;
     s_code[team][lane] = nb0 >= 0 ? cd0 : 0;
   }
-#pragma unroll
-  for (int p = 0; p < GSP; p++)
-    if (active && lane + p * T < GS) s_geo[team][lane + p * T] = gv[p];
+  if (active && lane < 2 * NF) s_nrm[team][lane] = nv;
   __syncthreads();
 
   const int j = lane;
   const bool node_lane = active && lane < ND;
+  const int jx = TRI ? 0 : j % N, jy = TRI ? 0 : j / N;
   double lmax = 0.0;
-  bool bad = false;
+  double idet = 0.0;  // inverse mass at this node: 1 / det J (triangles), 1 / (w_j det J)
+  double mk = 0.0;    // the node's weight in the element mean, up to a factor per element
 
-  // ---- volume: nodal flux, contravariant components
+  // ---- volume: nodal flux, contravariant components. Edge f runs along
+  // (-n_1, n_0) of its area normal n.
   if (!A.face_only && node_lane) {
+    const double* n = s_nrm[team];
+    double J0, J1, J2, J3;  // dx/dxi, dx/deta, dy/dxi, dy/deta
+    double wj = 1.0;
+    if constexpr (TRI) {
+      mk = tb.mhat[j];
+      J0 = -n[1];
+      J2 = n[0];
+      J1 = n[5];
+      J3 = -n[4];
+    } else {
+      const double x = tb.x[jx], y = tb.x[jy];
+      wj = tb.w[jx] * tb.w[jy];
+      J0 = (1 - y) * -n[1] + y * n[5];
+      J2 = (1 - y) * n[0] + y * -n[4];
+      J1 = (1 - x) * n[7] + x * -n[3];
+      J3 = (1 - x) * -n[6] + x * n[2];
+    }
+    const double det = J0 * J3 - J1 * J2;
+    idet = recip(wj * det);
+    if constexpr (!TRI) mk = wj * det;
+    const double adj[4] = {wj * J3, wj * -J1, wj * -J2, wj * J0};
     double st[NEQ];
 #pragma unroll
     for (int v = 0; v < NEQ; v++) st[v] = s_u[team][v][j];
     const SidePrim<2> q = side_prim<2>(st, g);
-    lmax = sqrt_ws(q.m2) * q.inv + side_sound<2>(st, q, g);
-    const double* adj = TRI ? &s_geo[team][C::G_ADJ] : &s_geo[team][C::G_ADJ + 4 * j];
+    if (!A.no_lambda) lmax = sqrt_ws(q.m2) * q.inv + side_sound<2>(st, q, g);
 #pragma unroll
     for (int r = 0; r < 2; r++) {
       const double a0 = adj[r * 2 + 0], a1 = adj[r * 2 + 1];
@@ -88,46 +172,112 @@ __device__ __forceinline__ void dense_rhs_block(const RhsArgs& A, const SchemePa
       s_g[team][r][3][j] = mai * (st[3] + q.p);
     }
   }
-  // ---- face points: traces, Riemann solve, weighted flux
-  for (int it = lane; it < NPT; it += T) {
-    if (!active) break;
-    const int f = it / NQ, q = it - f * NQ;
-    const int nb = s_nb[team][f];
+  // ---- traces
+  if constexpr (TRI) {
+#pragma unroll
+    for (int p = 0; p < RP; p++) {
+      if (rnb[p] >= 0) {
+#pragma unroll
+        for (int k = 0; k < ND; k++) s_t[team][(lane + p * T) * ND + k] = row[p][k];
+      }
+    }
+  } else {
+    // local faces 0..3: bottom, right, top, left; face f is normal to axis
+    // r = (f + 1) % 2, on its side c
+#pragma unroll
+    for (int p = 0; p < RP; p++) {
+      const int it = lane + p * T;
+      if (active && it < C::ROWS) {
+        const int f = it / NEQ, v = it % NEQ;
+        const double* uo = &s_u[team][v][0];
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          if (s == 1 && rnb[p] < 0) break;
+          const int fs = s == 0 ? f : (s_code[team][f] & 7);
+          const bool along_x = (fs & 1) == 0;  // the face runs along x (normal to y)
+          const int c = (fs == 1 || fs == 2) ? 1 : 0;
+          double tr[N];
+#pragma unroll
+          for (int a = 0; a < N; a++) {
+            double t = 0.0;
+#pragma unroll
+            for (int k = 0; k < N; k++) {
+              const double uv = s == 0 ? uo[along_x ? a + N * k : k + N * a]
+                                       : (along_x ? row[p][a + N * k] : row[p][k + N * a]);
+              t += tb.E[c][k] * uv;
+            }
+            tr[a] = t;
+          }
+#pragma unroll
+          for (int i = 0; i < NQ; i++) {
+            double t = 0.0;
+#pragma unroll
+            for (int a = 0; a < N; a++) t += tb.B[i][a] * tr[a];
+            s_t[team][((s * NF + f) * NQ + i) * NEQ + v] = t;
+          }
+        }
+      }
+    }
+  }
+  __syncthreads();
+
+  // ---- face points: Riemann solve, weighted flux; one lane per point. The
+  // point index i counts along the face's axis (quadrilaterals) or edge
+  if (active) {
+    const int f = lane / NQ, i = lane - f * NQ;
+    const int nb = s_nb[team][f], code = s_code[team][f];
+    const int fn = code & 7;
+    // edge parameter, mirrored on the neighbour when its edge runs the other way
+    const int q = TRI || f < 2 ? i : NQ - 1 - i;
+    const int q2 = ((code >> 3) & 2) ? NQ - 1 - q : q;
     double um[NEQ], up[NEQ], fl[NEQ];
+    if constexpr (TRI) {
+      double ph[ND];
 #pragma unroll
-    for (int v = 0; v < NEQ; v++) {
-      double t = 0.0;
-#pragma unroll
-      for (int k = 0; k < ND; k++) t += s_u[team][v][k] * tb.Phi[f][q][k];
-      um[v] = t;
-    }
-    double an[2];
-    double factor = -1.0;
-    bool ok = true;
-    double lam = 0.0;
-    const int code = s_code[team][f];
-    const bool elem1 = nb < 0 || ((code >> 6) & 1);
-    if (elem1) {
-      an[0] = s_geo[team][C::G_NRM + 2 * f];
-      an[1] = s_geo[team][C::G_NRM + 2 * f + 1];
-    } else {
-      const int fn = code & 7;
-      an[0] = A.geo[(int64_t)(C::G_NRM + 2 * fn) * NE + nb];
-      an[1] = A.geo[(int64_t)(C::G_NRM + 2 * fn + 1) * NE + nb];
-    }
-    const double normag = sqrt_ws(an[0] * an[0] + an[1] * an[1]);
-    const double inv = 1.0 / norml2_scaled<2>(an);
-    const double nrm[2] = {an[0] * inv, an[1] * inv};
-    if (!BC || nb >= 0) {
-      const int fn = code & 7;
-      const int q2 = ((code >> 3) & 2) ? NQ - 1 - q : q;
-      const double* xn = A.x + (int64_t)nb * ND;
+      for (int k = 0; k < ND; k++) ph[k] = tb.Phi[f][q][k];
 #pragma unroll
       for (int v = 0; v < NEQ; v++) {
         double t = 0.0;
 #pragma unroll
-        for (int k = 0; k < ND; k++) t += xn[v * NDOFS + k] * tb.Phi[fn][q2][k];
-        up[v] = t;
+        for (int k = 0; k < ND; k++) t += s_u[team][v][k] * ph[k];
+        um[v] = t;
+      }
+    } else {
+#pragma unroll
+      for (int v = 0; v < NEQ; v++) um[v] = s_t[team][(f * NQ + i) * NEQ + v];
+    }
+    const bool elem1 = nb < 0 || ((code >> 6) & 1);
+    double an[2];
+    if (elem1 || A.aligned) {
+      // Elem1's normal; where every shared edge has the same two end points the
+      // neighbour's is the exact negative of the own one
+      an[0] = elem1 ? s_nrm[team][2 * f] : -s_nrm[team][2 * f];
+      an[1] = elem1 ? s_nrm[team][2 * f + 1] : -s_nrm[team][2 * f + 1];
+    } else {
+      an[0] = A.geo[(int64_t)(C::G_NRM + 2 * fn) * NE + nb];
+      an[1] = A.geo[(int64_t)(C::G_NRM + 2 * fn + 1) * NE + nb];
+    }
+    const double normag = sqrt_ws(an[0] * an[0] + an[1] * an[1]);
+    const double inv = recip(normag);
+    const double nrm[2] = {an[0] * inv, an[1] * inv};
+    bool ok = true;
+    double lam = 0.0;
+    if (!BC || nb >= 0) {
+      if constexpr (TRI) {
+        double ph[ND];
+#pragma unroll
+        for (int k = 0; k < ND; k++) ph[k] = tb.Phi[fn][q2][k];
+#pragma unroll
+        for (int v = 0; v < NEQ; v++) {
+          double t = 0.0;
+#pragma unroll
+          for (int k = 0; k < ND; k++) t += s_t[team][(f * NEQ + v) * ND + k] * ph[k];
+          up[v] = t;
+        }
+      } else {
+        const int i2 = fn < 2 ? q2 : NQ - 1 - q2;
+#pragma unroll
+        for (int v = 0; v < NEQ; v++) up[v] = s_t[team][((NF + f) * NQ + i2) * NEQ + v];
       }
       double sL[NEQ], sR[NEQ];
 #pragma unroll
@@ -135,7 +285,6 @@ __device__ __forceinline__ void dense_rhs_block(const RhsArgs& A, const SchemePa
         sL[v] = elem1 ? um[v] : up[v];
         sR[v] = elem1 ? up[v] : um[v];
       }
-      if (!elem1) factor = 1.0;
       lam = riemann_t<2, RS>(g, sL, sR, nrm, fl, ok);
     } else if constexpr (BC) {
       const int slot = -1 - nb;
@@ -150,86 +299,28 @@ __device__ __forceinline__ void dense_rhs_block(const RhsArgs& A, const SchemePa
       }
     }
     if (!ok || lam < 0.0) {
-      if (!bad) {
-        const int64_t other = nb >= 0 ? (int64_t)nb : -1;
-        const bool mine = factor < 0.0;
-        const bool nf = nonfinite_nodes(A.x, NDOFS, e, ND, NEQ) || nonfinite_nodes(A.x, NDOFS, other, ND, NEQ);
-        flag_error(A.err, mine ? e : other, mine ? other : e, f, nf ? kErrNonFinite : kErrUnphysical);
-      }
-      bad = true;
+      const int64_t other = nb >= 0 ? (int64_t)nb : -1;
+      const bool nf = nonfinite_nodes(A.x, NDOFS, e, ND, NEQ) || nonfinite_nodes(A.x, NDOFS, other, ND, NEQ);
+      flag_error(A.err, elem1 ? e : other, elem1 ? other : e, f, nf ? kErrNonFinite : kErrUnphysical);
     } else {
       lmax = lam > lmax ? lam : lmax;
     }
-    const double wgt = factor * tb.wq[q] * normag;
+    double wgt = elem1 ? -normag : normag;
+    if constexpr (!TRI) wgt *= tb.wq[i];
 #pragma unroll
-    for (int v = 0; v < NEQ; v++) s_f[team][it][v] = fl[v] * wgt;
+    for (int v = 0; v < NEQ; v++) s_f[team][lane][v] = fl[v] * wgt;
   }
-  __syncthreads();
 
-  // ---- node lanes: volume contraction + lift
-  double z[NEQ];
-#pragma unroll
-  for (int v = 0; v < NEQ; v++) z[v] = 0.0;
-  if (node_lane) {
-    if (!A.face_only) {
-#pragma unroll
-      for (int r = 0; r < 2; r++)
-#pragma unroll
-        for (int k = 0; k < ND; k++) {
-          const double kk = tb.K[r][j][k];
-#pragma unroll
-          for (int v = 0; v < NEQ; v++) z[v] += kk * s_g[team][r][v][k];
-        }
-    }
-#pragma unroll
-    for (int f = 0; f < NF; f++)
-#pragma unroll
-      for (int q = 0; q < NQ; q++) {
-        const double ph = tb.Phi[f][q][j];
-#pragma unroll
-        for (int v = 0; v < NEQ; v++) z[v] += s_f[team][f * NQ + q][v] * ph;
-      }
-  }
   if (!A.face_only) {
     __syncthreads();
-    if (node_lane) {
-#pragma unroll
-      for (int v = 0; v < NEQ; v++) s_g[team][0][v][j] = z[v];
-    }
-    __syncthreads();
-    // ---- inverse mass and stage epilogue
+    // ---- node lanes: volume contraction, lift, inverse mass and stage epilogue
     double outv[NEQ];
-    double mk = 0.0;
     if (node_lane) {
-      double y[NEQ];
-#pragma unroll
-      for (int v = 0; v < NEQ; v++) y[v] = 0.0;
-      if (TRI) {
-        const double idet = recip(s_geo[team][C::G_DET]);
-#pragma unroll
-        for (int k = 0; k < ND; k++) {
-          const double mi = tb.Minv[j][k];
-#pragma unroll
-          for (int v = 0; v < NEQ; v++) y[v] += mi * s_g[team][0][v][k];
-        }
-#pragma unroll
-        for (int v = 0; v < NEQ; v++) y[v] *= idet;
-        mk = tb.mhat[j] * s_geo[team][C::G_DET];
-      } else {
-#pragma unroll
-        for (int k = 0; k < ND; k++) {
-          const double mi = s_geo[team][C::G_MINV + j * ND + k];
-#pragma unroll
-          for (int v = 0; v < NEQ; v++) y[v] += mi * s_g[team][0][v][k];
-        }
-        mk = s_geo[team][C::G_MW + j];
-      }
-      const double dtm = A.dt_inst ? A.dt_inst[ins] : 1.0;
-      // every base is loaded before the first store (an output may be its own base)
+      // every base is loaded before the first store (an output may be its own
+      // base) and in flight during the contraction; without one the base is the
+      // stage input
       const int64_t i0 = e * ND + j;
-      double u0[NEQ];
-#pragma unroll
-      for (int v = 0; v < NEQ; v++) u0[v] = s_u[team][v][j];
+      const double dtm = A.dt_inst ? A.dt_inst[ins] : 1.0;
       double base[4][NEQ];
 #pragma unroll
       for (int m = 0; m < 4; m++) {
@@ -238,11 +329,59 @@ __device__ __forceinline__ void dense_rhs_block(const RhsArgs& A, const SchemePa
           bp += i0;
 #pragma unroll
           for (int v = 0; v < NEQ; v++) base[m][v] = bp[v * NDOFS];
-        } else {
-#pragma unroll
-          for (int v = 0; v < NEQ; v++) base[m][v] = u0[v];
         }
       }
+      double y[NEQ];
+#pragma unroll
+      for (int v = 0; v < NEQ; v++) y[v] = 0.0;
+      if constexpr (TRI) {
+#pragma unroll
+        for (int r = 0; r < 2; r++)
+#pragma unroll
+          for (int k = 0; k < ND; k++) {
+            const double kk = tb.KM[r][j][k];
+#pragma unroll
+            for (int v = 0; v < NEQ; v++) y[v] += kk * s_g[team][r][v][k];
+            if (k % 2 == 1) hold();
+          }
+#pragma unroll
+        for (int pt = 0; pt < NPT; pt++) {
+          const double ph = tb.LM[pt][j];
+#pragma unroll
+          for (int v = 0; v < NEQ; v++) y[v] += s_f[team][pt][v] * ph;
+          if (pt % 3 == 2) hold();
+        }
+      } else {
+#pragma unroll
+        for (int a = 0; a < N; a++) {
+          const double dx = tb.D[a][jx], dy = tb.D[a][jy];
+#pragma unroll
+          for (int v = 0; v < NEQ; v++)
+            y[v] += dx * s_g[team][0][v][a + N * jy] + dy * s_g[team][1][v][jx + N * a];
+          hold();
+        }
+#pragma unroll
+        for (int f = 0; f < NF; f++) {
+          const int c = (f == 1 || f == 2) ? 1 : 0;
+          const int ja = (f & 1) == 0 ? jx : jy;  // the node's index along the face, and across it
+          const double ec = tb.E[c][(f & 1) == 0 ? jy : jx];
+          double L[NEQ];
+#pragma unroll
+          for (int v = 0; v < NEQ; v++) L[v] = 0.0;
+#pragma unroll
+          for (int i = 0; i < NQ; i++) {
+            const double b = tb.B[i][ja];
+#pragma unroll
+            for (int v = 0; v < NEQ; v++) L[v] += s_f[team][f * NQ + i][v] * b;
+          }
+#pragma unroll
+          for (int v = 0; v < NEQ; v++) y[v] += L[v] * ec;
+          hold();
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < NEQ; v++) y[v] *= idet;
+      pin<NEQ>(y);
 #pragma unroll
       for (int v = 0; v < NEQ; v++) outv[v] = 0.0;
 #pragma unroll
@@ -251,9 +390,11 @@ __device__ __forceinline__ void dense_rhs_block(const RhsArgs& A, const SchemePa
           double* op = A.outs[m].out + i0;
           const double cf = A.outs[m].coef * dtm;
           const double wb = A.outs[m].wb, wi = A.outs[m].wi;
+          const bool own = A.outs[m].base == nullptr;
 #pragma unroll
           for (int v = 0; v < NEQ; v++) {
-            const double o = wi == 0.0 ? base[m][v] + cf * y[v] : wb * base[m][v] + wi * (u0[v] + cf * y[v]);
+            const double u0 = s_u[team][v][j], b = own ? u0 : base[m][v];
+            const double o = wi == 0.0 ? b + cf * y[v] : wb * b + wi * (u0 + cf * y[v]);
             op[v * NDOFS] = o;
             if (m == A.means_of) outv[v] = o;
           }
@@ -266,7 +407,7 @@ __device__ __forceinline__ void dense_rhs_block(const RhsArgs& A, const SchemePa
       }
     }
     if (A.means) {
-      __syncthreads();
+      __syncthreads();  // the contraction's reads of s_g are done
       if (node_lane) {
 #pragma unroll
         for (int v = 0; v < NEQ; v++) s_g[team][1][v][j] = outv[v];
@@ -275,6 +416,7 @@ __device__ __forceinline__ void dense_rhs_block(const RhsArgs& A, const SchemePa
       __syncthreads();
       if (active && lane < NEQ) {
         double s = 0.0, ms = 0.0;
+#pragma unroll
         for (int k = 0; k < ND; k++) {
           const double w = s_g[team][0][0][k];
           s += w * s_g[team][1][lane][k];
@@ -284,22 +426,20 @@ __device__ __forceinline__ void dense_rhs_block(const RhsArgs& A, const SchemePa
       }
     }
   }
-  // ---- max wave speed: per instance slot
-  for (int off = T / 2; off > 0; off >>= 1) {
-    const double o = __shfl_xor(lmax, off, 64);
-    lmax = o > lmax ? o : lmax;
-  }
-  const int64_t elast = e0 + EPB - 1 < NE ? e0 + EPB - 1 : NE - 1;
-  const bool uniform = !A.inst || (e0 < NE && A.inst[e0] == A.inst[elast]);
-  if (uniform) {
-    for (int off = 32; off >= T; off >>= 1) {
-      const double o = __shfl_xor(lmax, off, 64);
-      lmax = o > lmax ? o : lmax;
+  // ---- max wave speed: one atomic per wave, or per lane where the block's
+  // elements belong to different instances
+  if (!A.no_lambda) {
+    const int64_t elast = e0 + EPB - 1 < NE ? e0 + EPB - 1 : NE - 1;
+    const int i0 = A.inst ? A.inst[e0] : 0;
+    if (!A.inst || i0 == A.inst[elast]) {
+      for (int off = 32; off > 0; off >>= 1) {
+        const double o = __shfl_xor(lmax, off, 64);
+        lmax = o > lmax ? o : lmax;
+      }
+      if (tid == 0) atomic_max_pos(A.lam + i0, lmax);
+    } else if (active) {
+      atomic_max_pos(A.lam + ins, lmax);
     }
-    const int i0 = A.inst && e0 < NE ? A.inst[e0] : 0;
-    if (tid == 0) atomic_max_pos(A.lam + (A.inst ? i0 : 0), lmax);
-  } else if (lane == 0 && active) {
-    atomic_max_pos(A.lam + ins, lmax);
   }
   __syncthreads();  // LDS is reused by the next work block
 }
@@ -308,8 +448,10 @@ __device__ __forceinline__ void dense_rhs_block(const RhsArgs& A, const SchemePa
 template <int GEOM, int P, int RS, bool BC>
 __global__ __launch_bounds__(64, 3) void dense_rhs_kernel(const RhsArgs A, const SchemeParams g,
                                                        const double* __restrict__ gtab, int64_t nvb) {
-  __shared__ DenseTab<GEOM, P> tb;
-  stage_dense<GEOM, P>(tb, gtab);
+  __shared__ __attribute__((aligned(16))) DenseRhsTab<GEOM, P> tb;
+  CopyRegs<sizeof(DenseRhsTab<GEOM, P>) / sizeof(double), 64> tbr;
+  tbr.load(gtab, threadIdx.x);
+  tbr.store(reinterpret_cast<double*>(&tb), threadIdx.x);
   __syncthreads();
   for (int64_t vb = blockIdx.x; vb < nvb; vb += gridDim.x) {
     // keep table reads inside the iteration (hoisted, they would hold registers across the loop)
@@ -561,6 +703,14 @@ int dense_table_size(int geom, int p) {
   return 0;
 }
 
+int dense_rhs_table_size(int geom, int p) {
+#define X(G, PP) \
+  if (geom == G && p == PP) return (int)(sizeof(DenseRhsTab<G, PP>) / sizeof(double));
+  RKDG_DENSE_CASES(X)
+#undef X
+  return 0;
+}
+
 int dense_geo_size(int geom, int p) {
 #define X(G, PP) \
   if (geom == G && p == PP) return DC<G, PP>::GSIZE;
@@ -571,7 +721,7 @@ int dense_geo_size(int geom, int p) {
 
 template <int G, int PP, int RS>
 hipError_t dense_rhs_rs(const RhsArgs& a, const SchemeParams& g, const double* t, bool bc, hipStream_t s) {
-  using C = DC<G, PP>;
+  using C = RC<G, PP>;
   const int64_t nvb = (a.NE + C::EPB - 1) / C::EPB;
   const int64_t grid = a.grid_cap > 0 && a.grid_cap < nvb ? a.grid_cap : nvb;
   if (bc) dense_rhs_kernel<G, PP, RS, true><<<(unsigned)grid, C::BLOCK, 0, s>>>(a, g, t, nvb);

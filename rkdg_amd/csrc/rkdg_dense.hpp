@@ -49,6 +49,28 @@ struct DenseTab {
   double PhiV[C::NV][C::ND];        // reference vertices (last hope)
 };
 
+// Tables of the right-hand side. Triangles: the volume and lift operators with
+// the reference inverse mass (and the face weights) folded in,
+// KM[r] = Mhat^-1 K[r] and LM[f*NQ+q][j] = wq[q] sum_k Mhat^-1[j][k] Phi[f][q][k].
+// Quadrilaterals: the 1D tables of the tensor-product basis (TensorTables).
+template <int GEOM, int P, bool TRI = DC<GEOM, P>::TRI>
+struct DenseRhsTab {
+  using C = DC<GEOM, P>;
+  double KM[2][C::ND][C::ND];
+  double Phi[C::NF][C::NQ][C::ND];
+  double LM[C::NPT][C::ND];
+  double mhat[C::ND];
+};
+template <int GEOM, int P>
+struct DenseRhsTab<GEOM, P, false> {
+  static constexpr int N = P + 1, NQ = DC<GEOM, P>::NQ;
+  double x[N], w[N];
+  double D[N][N];
+  double E[2][N];
+  double B[NQ][N];
+  double wq[NQ];
+};
+
 template <int GEOM, int P>
 __device__ __forceinline__ void stage_dense(DenseTab<GEOM, P>& d, const double* s) {
   constexpr int n = sizeof(DenseTab<GEOM, P>) / sizeof(double);

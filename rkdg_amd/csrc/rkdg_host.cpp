@@ -171,6 +171,7 @@ struct rkdg_ctx {
   TensorTables* d_tb = nullptr;
   int dense = 0;                 // 1: dense small-element kernels (triangles, bilinear quads)
   double* d_dtab = nullptr;      // dense reference tables
+  double* d_rtab = nullptr;      // tables of the dense right-hand side (DenseRhsTab)
   double* d_shu_coef = nullptr;  // Shu indicator: extrapolation weights [(nf+1)*nd][NE]
   int8_t* d_shu_flag = nullptr;  // Shu indicator: troubled elements of the last pass
   std::vector<double> ref_nodes; // reference node coordinates [nd][dim] (dense path)
@@ -214,7 +215,7 @@ struct rkdg_ctx {
   int* d_nce = nullptr;
   int* d_ncptr = nullptr;
   int* d_ncitem = nullptr;
-  int aligned = 0;               // tensor mesh: every interior face joins (r, c) to (r, 1-c), identity orientation
+  int aligned = 0;               // RhsArgs::aligned
   int grid_cap = 0;              // persistent grid of the dense right-hand-side kernel
   std::vector<int64_t> inst_off; // [count+1] element offsets
   int* d_inst = nullptr;         // [NE] element -> instance
@@ -281,6 +282,7 @@ void free_ctx(rkdg_ctx* c) {
   dfree(c->d_fbuf);
   dfree(c->d_tb);
   dfree(c->d_dtab);
+  dfree(c->d_rtab);
   dfree(c->d_shu_coef);
   if (c->d_shu_flag) (void)hipFree(c->d_shu_flag);
   for (auto& p : c->d_stage) dfree(p);
@@ -594,6 +596,38 @@ int build_dense(rkdg_ctx* c, const rkdg_mesh_desc* m) {
     for (int k = 0; k < nd; k++) PhiV[v * nd + k] = phi[k];
   }
 
+  // tables of the right-hand side, laid out exactly as DenseRhsTab<GEOM, P>
+  std::vector<double> rtab;
+  if (tri) {
+    for (int r = 0; r < 2; r++)
+      for (int j2 = 0; j2 < nd; j2++)
+        for (int k = 0; k < nd; k++) {
+          double t = 0.0;
+          for (int l = 0; l < nd; l++) t += Minv[j2 * nd + l] * K[(r * nd + l) * nd + k];
+          rtab.push_back(t);
+        }
+    rtab.insert(rtab.end(), Phi, Phi + nf * NQ * nd);
+    for (int pt = 0; pt < nf * NQ; pt++)
+      for (int j2 = 0; j2 < nd; j2++) {
+        double t = 0.0;
+        for (int l = 0; l < nd; l++) t += Minv[j2 * nd + l] * Phi[pt * nd + l];
+        rtab.push_back(wq[pt % NQ] * t);
+      }
+    rtab.insert(rtab.end(), mhat, mhat + nd);
+  } else {
+    const int N = p + 1;
+    rtab.insert(rtab.end(), gx1.begin(), gx1.end());
+    rtab.insert(rtab.end(), gw1.begin(), gw1.end());
+    for (int a = 0; a < N; a++)
+      for (int b = 0; b < N; b++) rtab.push_back(dlag(gx1.data(), N, b, gx1[a]));
+    for (int cc = 0; cc < 2; cc++)
+      for (int b = 0; b < N; b++) rtab.push_back(lag(gx1.data(), N, b, (double)cc));
+    for (int q = 0; q < NQ; q++)
+      for (int b = 0; b < N; b++) rtab.push_back(lag(gx1.data(), N, b, sq[q]));
+    rtab.insert(rtab.end(), wq.begin(), wq.end());
+  }
+  if ((int)rtab.size() != dense_rhs_table_size(m->geom, p)) return fail(RKDG_E_ARG, "dense table layout mismatch");
+
   // per-element geometry
   const int GS = dense_geo_size(m->geom, p);
   const int G_NRM = tri ? 5 : 4 * nd + nd * nd + nd;
@@ -715,6 +749,18 @@ int build_dense(rkdg_ctx* c, const rkdg_mesh_desc* m) {
     nbr[of.second.second * NE + of.second.first] = -1 - slot;
     c->n_bdr++;
   }
+  // a shared edge has the same two end points on both sides unless the mesh is
+  // periodic there: its two normals are then exact negatives of each other
+  c->aligned = 1;
+  for (int64_t e = 0; e < NE && c->aligned; e++)
+    for (int lf = 0; lf < nf; lf++) {
+      const int nb = nbr[(size_t)lf * NE + e];
+      if (nb < 0) continue;
+      const int fn = fcode[(size_t)lf * NE + e] & 7;
+      for (int d = 0; d < 2; d++)
+        if (c->geo_h[(size_t)(G_NRM + 2 * lf + d) * NE + e] != -c->geo_h[(size_t)(G_NRM + 2 * fn + d) * NE + nb])
+          c->aligned = 0;
+    }
   HIP_TRY(hipMalloc(&c->d_geo, sizeof(double) * GS * NE));
   HIP_TRY(hipMemcpy(c->d_geo, c->geo_h.data(), sizeof(double) * GS * NE, hipMemcpyHostToDevice));
   HIP_TRY(hipMalloc(&c->d_nbr, sizeof(int) * nf * NE));
@@ -724,6 +770,8 @@ int build_dense(rkdg_ctx* c, const rkdg_mesh_desc* m) {
   HIP_TRY(hipMemcpy(c->d_fcode, fcode.data(), sizeof(int) * nf * NE, hipMemcpyHostToDevice));
   HIP_TRY(hipMalloc(&c->d_dtab, sizeof(double) * tsize));
   HIP_TRY(hipMemcpy(c->d_dtab, tab.data(), sizeof(double) * tsize, hipMemcpyHostToDevice));
+  HIP_TRY(hipMalloc(&c->d_rtab, sizeof(double) * rtab.size()));
+  HIP_TRY(hipMemcpy(c->d_rtab, rtab.data(), sizeof(double) * rtab.size(), hipMemcpyHostToDevice));
   HIP_TRY(hipMalloc(&c->d_lam, sizeof(double) * 8 * c->count));
   HIP_TRY(hipMemset(c->d_lam, 0, sizeof(double) * 8 * c->count));
   HIP_TRY(hipMalloc(&c->d_err, sizeof(long long) * 4));
@@ -1553,7 +1601,7 @@ hipError_t rhs_launch(rkdg_ctx* c, const RhsArgs& a0) {
   auto pr = prof_begin(c, c->ev_rhs);
   hipError_t e;
   if (c->dense) {
-    e = launch_dense_rhs(c->geom, c->p, a, c->sp, c->d_dtab, c->n_bdr > 0, c->stream);
+    e = launch_dense_rhs(c->geom, c->p, a, c->sp, c->d_rtab, c->n_bdr > 0, c->stream);
   } else if (c->rb) {
     // two-colour form: the solver elements (every face flux once, the
     // receiver's share to fbuf), then the receivers (their share read back)
@@ -1614,7 +1662,7 @@ RhsArgs base_args(rkdg_ctx* c, const double* x) {
   a.bcp = c->d_bcp;
   a.grid_cap = c->grid_cap;
   a.order = c->dense ? nullptr : c->d_order;
-  a.aligned = c->dense ? 0 : c->aligned;
+  a.aligned = c->aligned;
   a.cgeo = c->d_cgeo;
   return a;
 }
@@ -1823,6 +1871,7 @@ int batch_step_launch(rkdg_ctx* c, double* x, int s, const double* a, const doub
     const double* in = i == 0 ? x : W[i];
     RhsArgs ra = base_args(c, in);
     ra.lam = c->d_lam + (int64_t)i * c->count;
+    ra.no_lambda = i < s - 1 ? 1 : 0;  // only the last stage's wave speeds are read
     ra.dt_inst = c->d_dtr;
     ra.active = c->d_active;
     int n = 0;

@@ -75,7 +75,8 @@ struct RhsArgs {
   int64_t nlist;       // number of elements in elist
   const int* fslot;    // [NE]: receiver slot of each element (its index in the receivers' elist)
   double* fbuf;        // [receivers][NF][NEQ][face nodes]: lifted face fluxes in the receiver's face frame
-  int aligned;         // tensor kernel: every interior face joins faces (r, c) and (r, 1-c), identity orientation
+  int aligned;         // tensor kernel: every interior face joins faces (r, c) and (r, 1-c), identity orientation;
+                       // dense kernel: the two edge normals of every interior face are exact negatives
   // Limiter applied on load (tensor kernel, role 0; both null otherwise): x
   // holds the unlimited stage value and the kernel works on the limited one,
   // mean + f (u - mean) per element and variable with f = lim_f[e] and
@@ -341,6 +342,7 @@ int tensor_elems_per_block(int dim, int p);  // elements per workgroup of the te
 // t points to the device copy of the dense reference tables
 bool dense_supported(int geom, int p);
 int dense_table_size(int geom, int p);  // doubles
+int dense_rhs_table_size(int geom, int p);  // doubles
 int dense_geo_size(int geom, int p);    // doubles per element
 hipError_t launch_dense_rhs(int geom, int p, const RhsArgs& a, const SchemeParams& g, const double* t,
                             bool has_bdr, hipStream_t s);

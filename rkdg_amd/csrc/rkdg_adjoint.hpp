@@ -319,7 +319,7 @@ RKDG_HD void riemann_vjp(const SchemeParams& g, const double* uL, const double* 
       f2[3] = u2 * (s2[3] + p2);
     }
     double SL, SR;
-    wave_speeds<2>(s1, s2, p1, p2, g, SL, SR);
+    wave_speeds<2>(s1, s2, side_prim<2>(s1, g), side_prim<2>(s2, g), g, SL, SR);
     double f1bar[NE2] = {0, 0, 0, 0}, f2bar[NE2] = {0, 0, 0, 0};
     double SLbar = 0.0, SRbar = 0.0;
     if constexpr (RS == RKDG_RS_LLF) {

@@ -890,6 +890,7 @@ static int scheme_params(const rkdg_scheme_desc* s, SchemeParams& g) {
   g.last_hope = s->last_hope;
   g.pow_nd = s->pow_nd;
   g.linearize = s->linearize ? 1 : 0;
+  derive_params(g);
   return RKDG_OK;
 }
 

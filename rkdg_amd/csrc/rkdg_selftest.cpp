@@ -29,6 +29,7 @@ SchemeParams params(const rkdg_scheme_desc* s) {
   g.limiter = s->limiter;
   g.last_hope = s->last_hope;
   g.pow_nd = s->pow_nd;
+  derive_params(g);
   return g;
 }
 

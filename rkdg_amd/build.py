@@ -17,6 +17,8 @@ BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "librkdg.so")
 SOURCES = ["rkdg_tensor.hip", "rkdg_dense.hip", "rkdg_batch.hip", "rkdg_adjoint.hip", "rkdg_noalloc.hip", "rkdg_io.hip", "rkdg_shu.hip",
            "rkdg_nc.hip", "rkdg_host.cpp", "rkdg_selftest.cpp"]
+# sources built as several objects: macro and number of parts (numbered from 0)
+PARTS = {"rkdg_tensor.hip": ("RKDG_TENSOR_PART", 5)}
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -40,9 +42,12 @@ def build(verbose: bool = False) -> str:
     objs = []
     cmds = []
     for src in SOURCES:
-        obj = os.path.join(BUILD, src + ".o")
-        objs.append(obj)
-        cmds.append([HIPCC, *FLAGS, "-c", os.path.join(CSRC, src), "-o", obj])
+        macro, n = PARTS.get(src, (None, 1))
+        for k in range(n):
+            obj = os.path.join(BUILD, f"{src}.{k}.o" if macro else src + ".o")
+            objs.append(obj)
+            cmds.append([HIPCC, *FLAGS, *([f"-D{macro}={k}"] if macro else []), "-c", os.path.join(CSRC, src),
+                         "-o", obj])
     with ThreadPoolExecutor(max_workers=len(cmds)) as ex:
         list(ex.map(lambda c: _run(c, verbose), cmds))
     tmp = LIB + ".tmp"

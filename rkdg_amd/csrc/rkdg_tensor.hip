@@ -184,6 +184,7 @@ __global__ __launch_bounds__(64, ROLE == 1 ? 4 : 1) void tensor_rhs_kernel(const
   __shared__ double s_geo[EPB][GD];
   __shared__ int s_nb[ES][NF];                // by MFEM local face
   __shared__ int s_code[ES][NF];
+  __shared__ int s_bad[ES];                   // lowest face index 2 r + c whose flux failed
   __shared__ int s_slot[ROLE == 1 ? EPB : 1][NF];      // receiver slot of each face's neighbour
   __shared__ double s_fb[ROLE == 2 ? EPB : 1][ROLE == 2 ? FB : 1];  // receivers: [lf][v][face node]
 
@@ -277,6 +278,7 @@ __global__ __launch_bounds__(64, ROLE == 1 ? 4 : 1) void tensor_rhs_kernel(const
     s_nrm[team][f][DIM] = sign * nmag;
     s_nrm[team][f][DIM + 1] = 0.5 * recip(sqrt_ws(nu2));
   }
+  if (SOLVE && lane == 0 && team < ES) s_bad[team] = NF;
   tbr.store(reinterpret_cast<double*>(&tb), tid);
   if (lim_load) {
 #pragma unroll
@@ -369,7 +371,6 @@ __global__ __launch_bounds__(64, ROLE == 1 ? 4 : 1) void tensor_rhs_kernel(const
     // ---- face terms, one axis at a time. Phases per axis r: points(r) |
     // lift(r) + traces(r+1) | node accumulation(r) + points(r+1) ..., so each
     // axis costs two barriers.
-    bool bad = false;
     // Table values that depend on the lane but not on the axis, read from LDS
     // once (the phases below are one pass of the team when ONE_PASS; otherwise
     // they read the tables per item).
@@ -540,16 +541,8 @@ __global__ __launch_bounds__(64, ROLE == 1 ? 4 : 1) void tensor_rhs_kernel(const
             for (int v = 0; v < NEQ; v++) fl[v] = 0.0;
           }
         }
-        if (!ok || lam < 0.0) {
-          if (!bad) {
-            const bool nf = nonfinite_nodes(A.x, NDOFS, e, ND, NEQ) || nonfinite_nodes(A.x, NDOFS, nb, ND, NEQ);
-            flag_error(A.err, factor < 0.0 ? e : nb, factor < 0.0 ? (nb >= 0 ? nb : -1) : e, lf,
-                       nf ? kErrNonFinite : kErrUnphysical);
-          }
-          bad = true;
-        } else {
-          lmax = lam > lmax ? lam : lmax;
-        }
+        if (!ok || lam < 0.0) atomicMin(&s_bad[team], f);  // classified and reported at the end
+        else lmax = lam > lmax ? lam : lmax;
         const double wgt = (ONE_PASS ? wq2 : (DIM == 3 ? tb.wq[qi] * tb.wq[qj] : tb.wq[qi])) * snm;  // flux sign * w_q * |n|
   #pragma unroll
         for (int v = 0; v < NEQ; v++) work[(c * NEQ + v) * RW + q] = fl[v] * wgt;
@@ -758,75 +751,149 @@ __global__ __launch_bounds__(64, ROLE == 1 ? 4 : 1) void tensor_rhs_kernel(const
     }
     if (tid == 0) atomic_max_pos(A.lam, lmax);
   }
-}
 
-// ---------------------------------------------------------------------------
-// element means (Averager::computeMeanValues): one team per element, lanes on
-// nodes (coalesced loads), sum_k w_k u_k / sum_k w_k by a shuffle reduction
-// over the team (det J is constant on an affine element and cancels)
-template <int DIM, int P>
-__global__ __launch_bounds__(64) void tensor_means_kernel(const MeansArgs A,
-                                                          const TensorTables* __restrict__ gtb) {
-  using C = TC<DIM, P>;
-  constexpr int N = C::N, ND = C::ND, NEQ = C::NEQ, T = C::T, EPB = C::EPB;
-  const int tid = threadIdx.x;
-  const int team = tid / T, lane = tid % T;
-  const int64_t NE = A.NE;
-  const int64_t NDOFS = NE * ND;
-  const int64_t e = (int64_t)blockIdx.x * EPB + team;
-  const bool on = e < NE && lane < ND;
-  double wk = 0.0, s[NEQ];
-#pragma unroll
-  for (int v = 0; v < NEQ; v++) s[v] = on ? A.x[v * NDOFS + e * ND + lane] : 0.0;
-  if (on) {
-    if (DIM == 3 && A.cgeo) {
-      // curved hexahedra: the integrals of the basis (Averager)
-      wk = A.cgeo[e * CurvedLayout<P>::size + CurvedLayout<P>::mw + lane];
-    } else {
-      wk = gtb->w[lane % N] * gtb->w[(lane / N) % N];
-      if (DIM == 3) wk *= gtb->w[lane / (N * N)];
+  // ---- a failed flux: the element pair, and whether a node of either is not
+  // finite (the input is not among the outputs, so it is still there). Here, at
+  // the end, the out-of-line scan costs the kernel no registers; a call among the
+  // face points kept every live value out of its way.
+  if constexpr (SOLVE) {
+    if (active && lane == 0 && s_bad[team] < NF) {
+      const int f = s_bad[team];
+      const int lf = lf_of<DIM>(f / 2, f % 2);
+      const int64_t nb = s_nb[team][lf] >= 0 ? s_nb[team][lf] : -1;
+      const bool elem1 = nb < 0 || ((s_code[team][lf] >> 6) & 1);
+      const bool nf = nonfinite_nodes(A.x, NDOFS, e, ND, NEQ) || nonfinite_nodes(A.x, NDOFS, nb, ND, NEQ);
+      flag_error(A.err, elem1 ? e : nb, elem1 ? nb : e, lf, nf ? kErrNonFinite : kErrUnphysical);
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// element means (Averager::computeMeanValues): sum_k w_k u_k / sum_k w_k (det J
+// is constant on an affine element and cancels). A workgroup stages the states
+// of EB elements through LDS with coalesced loads, then one lane per (element,
+// variable) forms the sum: bound by the read of the state. The tree of shuffles
+// over an element's lanes that this replaces issued ten per variable and ran at
+// half the copy rate (96^3 Q2 hexahedra: 300 -> 225 us; 63 x 65 x 61 just
+// after the limiter wrote them, from the caches: 97 -> 64 us).
+template <int DIM, int P>
+struct MC : TC<DIM, P> {
+  using C = TC<DIM, P>;
+  static constexpr int EB = C::ND <= 4 ? 128 : (C::ND <= 9 ? 64 : (C::ND <= 27 ? 32 : 16));
+  static constexpr int NDP = C::ND | 1;  // odd row length: the summing lanes hit different LDS banks
+};
+template <int DIM, int P>
+__global__ __launch_bounds__(256) void tensor_means_kernel(const MeansArgs A,
+                                                           const TensorTables* __restrict__ gtb) {
+  using C = MC<DIM, P>;
+  constexpr int N = C::N, ND = C::ND, NEQ = C::NEQ, EB = C::EB, NDP = C::NDP;
+  __shared__ double s_u[NEQ][EB][NDP];
+  __shared__ double s_w[DIM == 3 ? EB : 1][NDP];  // curved elements: each its own weights
+  const int tid = threadIdx.x;
+  const int64_t NE = A.NE, NDOFS = NE * ND;
+  const int64_t e0 = (int64_t)blockIdx.x * EB;
+  const int ne = NE - e0 < EB ? (int)(NE - e0) : EB;
+  const bool curved = DIM == 3 && A.cgeo != nullptr;
+  constexpr int LP = (EB * ND + 255) / 256;
 #pragma unroll
-  for (int v = 0; v < NEQ; v++) s[v] *= wk;
+  for (int p = 0; p < LP; p++) {
+    const int i = tid + 256 * p;
+    if (i < ne * ND) {
+      const int el = i / ND, k = i - el * ND;
 #pragma unroll
-  for (int off = T / 2; off > 0; off >>= 1) {
-    wk += __shfl_xor(wk, off, 64);
-#pragma unroll
-    for (int v = 0; v < NEQ; v++) s[v] += __shfl_xor(s[v], off, 64);
+      for (int v = 0; v < NEQ; v++) s_u[v][el][k] = A.x[v * NDOFS + e0 * ND + i];
+      if (curved) s_w[DIM == 3 ? el : 0][k] = A.cgeo[(e0 + el) * CurvedLayout<P>::size + CurvedLayout<P>::mw + k];
+    }
   }
-  if (e < NE && lane == 0) {
+  if (!curved && tid < ND) {
+    double w = gtb->w[tid % N] * gtb->w[(tid / N) % N];
+    if (DIM == 3) w *= gtb->w[tid / (N * N)];
+    s_w[0][tid] = w;
+  }
+  __syncthreads();
+  for (int i = tid; i < EB * NEQ; i += 256) {
+    const int v = i / EB, el = i - v * EB;
+    if (el < ne) {
+      const double* w = s_w[curved ? el : 0];
+      double s = 0.0, ws = 0.0;
 #pragma unroll
-    for (int v = 0; v < NEQ; v++) A.means[v * NE + e] = s[v] / wk;
+      for (int k = 0; k < ND; k++) {
+        s += w[k] * s_u[v][el][k];
+        ws += w[k];
+      }
+      A.means[v * NE + e0 + el] = s / ws;
+    }
   }
 }
 
 // ---------------------------------------------------------------------------
-// Limiter::update for one element per team: stencil bounds of the means over
-// the face neighbours, the indicator at two Gauss points per face direction of
-// every interior face, the limiter function, then LimiterMultiplier (with the
-// last-hope reset at the reference vertices) or LimiterFinDiff. Only the
-// indicator of the variable that decides is formed: the multiplier uses the
-// density's (minValues = yMin[rho], indicator_bj.cpp:193), FinDiff the last
-// variable's (limiter_findiff.cpp:7-8).
+// Limiter::update: stencil bounds of the means over the face neighbours, the
+// indicator at two Gauss points per face direction of every interior face, the
+// limiter function, then LimiterMultiplier (with the last-hope reset at the
+// reference vertices) or LimiterFinDiff. Only the indicator of the variable that
+// decides is formed: the multiplier uses the density's (minValues = yMin[rho],
+// indicator_bj.cpp:193), FinDiff the last variable's (limiter_findiff.cpp:7-8).
+//
+// One lane per vertex: T = 2^dim lanes per element, 64 / T elements per
+// wavefront. Lane (cx, cy, cz) evaluates the vertex and the one indicator point
+// of each of its three faces that lies next to that vertex (the two Gauss points
+// per direction go with the two ends), all from the element's nodes by sum
+// factorisation in registers; no intermediate goes through LDS, and every lane
+// works in every phase whatever the order. With a team of lanes per element
+// (32 for 27 nodes, of which the vertex phase used 8) the pass was bound by VALU
+// issue, 245 instructions per Q2 element; now it is bound by the read of the
+// state (factor pass at 96^3: 3.9 of the copy's 5 TB/s). 96^3 Q2: factor pass 385
+// -> 265 us, in-place pass 490 -> 415 us; 63,360 Q2 hexahedra 34 -> 23 us, 29,667
+// Q3 hexahedra 36 -> 29 us. An element whose factor is exactly 1 is not written.
 template <int DIM, int P>
-__global__ __launch_bounds__(64) void tensor_limit_kernel(const LimitArgs A, const SchemeParams g,
-                                                          const TensorTables* __restrict__ gtb) {
+struct LC : TC<DIM, P> {
   using C = TC<DIM, P>;
-  constexpr int N = C::N, ND = C::ND, NEQ = C::NEQ, NFN = C::NFN, NF = C::NF, NIP = C::NIP;
-  constexpr int T = C::T, EPB = C::EPB, BLOCK = C::BLOCK;
-  constexpr int NPT = NF * NIP;  // indicator points per element
-  constexpr int NVERT = C::NVERT;
+  static constexpr int T = C::NVERT;
+  static constexpr int EPB = 64 / T;
+  // LDS stride of an element: even (16-byte rows) and such that the elements of
+  // a wavefront, which read the same node at once, hit different banks
+  static constexpr int ROW = C::ND + (C::ND & 1);
+  static constexpr int want = DIM == 3 ? 4 : 2;
+  static constexpr int ES = C::NEQ * ROW + (32 + want - (C::NEQ * ROW) % 32) % 32;
+};
 
-  __shared__ TT<C::N, C::NQ> tb;
-  __shared__ double s_u[EPB][NEQ][ND];
-  __shared__ double s_tr[EPB][NF][NFN];   // traces of the deciding variable
-  constexpr int NB = DIM == 3 ? N : 1;
-  // last hope: every variable on the x faces interpolated to y = 0, 1: [cx][cy][v][z node]
-  __shared__ double s_ty[EPB][2][2][NEQ][NB];
-  __shared__ double s_mean[EPB][NEQ];  // the element's means
-  __shared__ double s_nbm[EPB][NF];    // deciding variable's means of the face neighbours (lowest)
-  __shared__ double s_nbh[EPB][NF];    // ... highest (several neighbours across a non-conforming face)
+template <int ctrl>
+__device__ __forceinline__ double dpp(double x) {
+  const uint64_t u = (uint64_t)__double_as_longlong(x);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, ctrl, 0xf, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), ctrl, 0xf, 0xf, true);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+// minimum (maximum) over the T = 4 or 8 lanes of an element: quad_perm by 1 and
+// 2, then row_half_mirror, which pairs the two quads of eight lanes
+template <int T>
+__device__ __forceinline__ double team_min(double x) {
+  double o = dpp<0xB1>(x);
+  x = o < x ? o : x;
+  o = dpp<0x4E>(x);
+  x = o < x ? o : x;
+  if (T == 8) {
+    o = dpp<0x141>(x);
+    x = o < x ? o : x;
+  }
+  return x;
+}
+template <int T>
+__device__ __forceinline__ double team_max(double x) {
+  return -team_min<T>(-x);
+}
+
+template <int DIM, int P>
+__global__ __launch_bounds__(64, 2) void tensor_limit_kernel(const LimitArgs A, const SchemeParams g,
+                                                          const TensorTables* __restrict__ gtb) {
+  using C = LC<DIM, P>;
+  constexpr int N = C::N, ND = C::ND, NEQ = C::NEQ, NF = C::NF, T = C::T, EPB = C::EPB;
+  constexpr int ROW = C::ROW, ES = C::ES;
+  constexpr int NZ = DIM == 3 ? N : 1;
+  __shared__ __attribute__((aligned(16))) double s_u[EPB * ES];  // [element][variable][node]
+  __shared__ double s_tab[4 * N];                                // E[2][N], BI[2][N]
+  __shared__ double s_mean[EPB][NEQ];
+  __shared__ double s_f[EPB];
 
   const int tid = threadIdx.x;
   const int team = tid / T, lane = tid % T;
@@ -840,28 +907,31 @@ __global__ __launch_bounds__(64) void tensor_limit_kernel(const LimitArgs A, con
     if (A.factor && active && lane == 0) A.factor[e] = 1.0;
     return;
   }
-  const int vsel = g.limiter == RKDG_LIM_FINDIFF ? NEQ - 1 : 0;
+  const bool multi = g.limiter == RKDG_LIM_MULTI, findiff = g.limiter == RKDG_LIM_FINDIFF;
+  const int vsel = findiff ? NEQ - 1 : 0;
 
   // every load of the setup is issued before the first LDS store
-  CopyRegs<sizeof(TT<N, C::NQ>) / sizeof(double), BLOCK> tbr;
-  tbr.load(gtb->packed, tid);
-  StateRegs<EPB, NEQ, ND, BLOCK> str;
-  str.load(A.x, NDOFS, e0, NE, tid);
-  // the element's means (lane v < NEQ) and the deciding variable's means of
-  // the face neighbours (lane lf < NF): one load instruction each, combined
-  // through LDS after the barrier (a wave-wide load per value would cost the
-  // memory pipeline 64 lanes for two distinct addresses)
+  constexpr int LP = (EPB * ND + 63) / 64;
+  const int nn = (int)((NE - e0 < EPB ? NE - e0 : EPB) * ND);  // nodes of this block's elements
+  double st[LP][NEQ];
+#pragma unroll
+  for (int p = 0; p < LP; p++) {
+    const int i = tid + 64 * p;
+#pragma unroll
+    for (int v = 0; v < NEQ; v++) st[p][v] = i < nn ? sbase(A.x + (v * NDOFS + e0 * ND))[(unsigned)i] : 1.0;
+  }
+  const double tabv = tid < 4 * N ? (tid < 2 * N ? gtb->E[tid / N][tid % N] : gtb->BI[tid / N - 2][tid % N]) : 0.0;
+  // the element's means (lane v < NEQ) and the deciding variable's means of the
+  // face neighbours (lane lf < NF): one load instruction each
   static_assert(NEQ <= T && NF <= T, "one lane per variable and per face");
   const bool ind_bj = g.indicator == RKDG_IND_BJ;
   const double mown = (active && lane < NEQ) ? A.means[lane * NE + e] : 0.0;
   const int nbl = (active && ind_bj && lane < NF) ? A.nbr[lane * NE + e] : -1;
-  double nml = nbl >= 0 ? A.means[vsel * NE + nbl] : 0.0;
-  double nmh = nml;  // a non-conforming face: the bounds over its neighbours
+  double nml = nbl >= 0 ? A.means[vsel * NE + nbl] : 1e300;
+  double nmh = nbl >= 0 ? nml : -1e300;
   bool has_nb = nbl >= 0;
-  if (A.ncnb && nbl <= kNcCode0) {
+  if (A.ncnb && nbl <= kNcCode0) {  // a non-conforming face: the bounds over its neighbours
     const int k = kNcCode0 - nbl;
-    nml = 1e300;
-    nmh = -1e300;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
       const int n = A.ncnb[4 * k + q];
@@ -873,8 +943,7 @@ __global__ __launch_bounds__(64) void tensor_limit_kernel(const LimitArgs A, con
     }
     has_nb = true;
   }
-  const unsigned long long nbb = __ballot(has_nb);
-  const int nbmask = (int)((nbb >> (team * T)) & ((1ull << NF) - 1ull));  // bit lf: face lf has a neighbour
+  const int nbmask = (int)(__ballot(has_nb) >> (team * T)) & ((1 << NF) - 1);  // bit lf: face lf has a neighbour
   // Venkatakrishnan eps^2 = (K h)^3 with h = |element|^(1/dim): h^3 = det J
   // (3D) or det J^(3/2) (2D) for affine elements
   double eps2 = 0.0;
@@ -883,120 +952,103 @@ __global__ __launch_bounds__(64) void tensor_limit_kernel(const LimitArgs A, con
     const double k3 = g.venkat_k * g.venkat_k * g.venkat_k;
     eps2 = k3 * (DIM == 3 ? dj : dj * sqrt(dj));
   }
-  tbr.store(reinterpret_cast<double*>(&tb), tid);
-  str.store(s_u, tid);
-  if (lane < NEQ) s_mean[team][lane] = mown;
-  if (lane < NF) {
-    s_nbm[team][lane] = nml;
-    s_nbh[team][lane] = nmh;
+  if (tid < 4 * N) s_tab[tid] = tabv;
+#pragma unroll
+  for (int p = 0; p < LP; p++) {
+    const int i = tid + 64 * p;
+    if (i < EPB * ND) {
+      const int el = i / ND, k = i - el * ND;
+#pragma unroll
+      for (int v = 0; v < NEQ; v++) s_u[el * ES + v * ROW + k] = st[p][v];
+    }
   }
+  if (lane < NEQ) s_mean[team][lane] = mown;
   __syncthreads();
   double mean[NEQ];
 #pragma unroll
   for (int v = 0; v < NEQ; v++) mean[v] = s_mean[team][v];
   // stencil bounds (cell + face neighbours) of the deciding variable's means
+  double msel = findiff ? mean[NEQ - 1] : mean[0];
   double mI = 1e9, MI = -1e9;
-  if (ind_bj && active) {
-    const double mv = mean[vsel];
-    mI = mv;
-    MI = mv;
-#pragma unroll
-    for (int lf = 0; lf < NF; lf++) {
-      if ((nbmask >> lf) & 1) {
-        const double a = s_nbm[team][lf], b = s_nbh[team][lf];
-        mI = a < mI ? a : mI;
-        MI = b > MI ? b : MI;
-      }
-    }
-  }
-
-  // normal-direction traces of the deciding variable on every face
   if (ind_bj) {
-    for (int it = lane; it < NF * NFN; it += T) {
-      if (!active) break;
-      const int f = it / NFN, fn = it - f * NFN;
-      const int r = f / 2, c = f % 2;
-      const int a = fn % N, b = fn / N;
-      int sk, sa, sb;
-      vstrides<DIM, N>(r, sk, sa, sb);
-      const double* uv = &s_u[team][vsel][a * sa + b * sb];
+    mI = team_min<T>(nml);
+    MI = team_max<T>(nmh);
+    mI = mI < msel ? mI : msel;
+    MI = MI > msel ? MI : msel;
+  }
+  // 1D weights of the lane's corner: E (the end of the axis) and BI (the Gauss
+  // point next to it)
+  const int cr[3] = {lane & 1, (lane >> 1) & 1, lane >> 2};
+  double wE[DIM][N], wB[DIM][N];
+#pragma unroll
+  for (int d = 0; d < DIM; d++)
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      wE[d][k] = s_tab[cr[d] * N + k];
+      wB[d][k] = s_tab[(2 + cr[d]) * N + k];
+    }
+  const double* ue = &s_u[team * ES];
+  // value of variable row u at the lane's vertex
+  auto at_vertex = [&](const double* u) {
+    double V = 0.0;
+#pragma unroll
+    for (int c = 0; c < NZ; c++) {
       double t = 0.0;
 #pragma unroll
-      for (int k = 0; k < N; k++) t += uv[k * sk] * tb.E[c][k];
-      s_tr[team][f][fn] = t;
+      for (int b = 0; b < N; b++) {
+        double r = 0.0;
+#pragma unroll
+        for (int a = 0; a < N; a++) r += u[a + N * (b + N * c)] * wE[0][a];
+        t += r * wE[1][b];
+      }
+      V += DIM == 3 ? t * wE[DIM - 1][c] : t;
     }
-  }
-  if constexpr (P == 1) {
-    // linearize: the multiplier and the last hope work on the element's linear
-    // reconstruction (the indicator above reads the state as it is)
-    if (g.linearize && g.limiter == RKDG_LIM_MULTI) {
-      double lin[NEQ];
-      const bool nl = active && lane < ND;
-      if (nl) {
-#pragma unroll
-        for (int v = 0; v < NEQ; v++) lin[v] = linearize_q1<DIM>(&s_u[team][v][0], mean[v], lane);
-      }
-      __syncthreads();
-      if (nl) {
-#pragma unroll
-        for (int v = 0; v < NEQ; v++) s_u[team][v][lane] = lin[v];
-      }
-      __syncthreads();
-    }
-  }
-  if (g.limiter == RKDG_LIM_MULTI && g.last_hope) {
-    // sum-factorised vertex values, first two directions: one lane per
-    // (x side cx, variable, z node b) forms the x-face traces of its row and
-    // interpolates them to y = 0 and y = 1
-    for (int it = lane; it < 2 * NEQ * NB; it += T) {
-      if (!active) break;
-      const int cx = it / (NEQ * NB), rem = it - cx * (NEQ * NB);
-      const int v = rem / NB, b = rem - v * NB;
-      double tr[N];
-#pragma unroll
-      for (int a = 0; a < N; a++) {
-        double t = 0.0;
-#pragma unroll
-        for (int k = 0; k < N; k++) t += s_u[team][v][vnode<DIM, N>(0, k, a, b)] * tb.E[cx][k];
-        tr[a] = t;
-      }
-#pragma unroll
-      for (int cy = 0; cy < 2; cy++) {
-        double tt = 0.0;
-#pragma unroll
-        for (int a = 0; a < N; a++) tt += tr[a] * tb.E[cy][a];
-        s_ty[team][cx][cy][v][b] = tt;
-      }
-    }
-  }
-  __syncthreads();
-
-  // indicator values at the points of interior faces
-  double ylane = 1e9;  // this lane's minimum over its indicator points
+    return V;
+  };
+  double vs[NEQ];  // the state at the vertex
+  double yr = 1e9;
   if (ind_bj) {
-    for (int it = lane; it < NPT; it += T) {
-      if (!active) break;
-      const int f = it / NIP, ip = it - f * NIP;
-      const int r = f / 2, c = f % 2;
-      const int lf = lf_of<DIM>(r, c);
-      double yc = 1e9;
-      if ((nbmask >> lf) & 1) {
-        const int pi = ip % 2, pj = ip / 2;
-        double u = 0.0;
-        if (DIM == 3) {
+    // the deciding variable at the vertex and at the lane's point on the face
+    // normal to each axis
+    double pt[DIM], V = 0.0;
 #pragma unroll
-          for (int b = 0; b < N; b++) {
-            double tt = 0.0;
+    for (int d = 0; d < DIM; d++) pt[d] = 0.0;
+    const double* u = ue + vsel * ROW;
 #pragma unroll
-            for (int a = 0; a < N; a++) tt += s_tr[team][f][a + N * b] * tb.BI[pi][a];
-            u += tt * tb.BI[pj][b];
-          }
-        } else {
+    for (int c = 0; c < NZ; c++) {
+      double tEB = 0.0, tBE = 0.0, tBB = 0.0, tEE = 0.0;
 #pragma unroll
-          for (int a = 0; a < N; a++) u += s_tr[team][f][a] * tb.BI[pi][a];
+      for (int b = 0; b < N; b++) {
+        double rE = 0.0, rB = 0.0;
+#pragma unroll
+        for (int a = 0; a < N; a++) {
+          const double x = u[a + N * (b + N * c)];
+          rE += x * wE[0][a];
+          rB += x * wB[0][a];
         }
-        const double diff = u - mean[vsel];
-        const double y = indicator_y(diff, mean[vsel], mI, MI);
+        tEB += rE * wB[1][b];
+        tBE += rB * wE[1][b];
+        tEE += rE * wE[1][b];
+        if (DIM == 3) tBB += rB * wB[1][b];
+      }
+      if (DIM == 3) {
+        pt[0] += tEB * wB[DIM - 1][c];
+        pt[1] += tBE * wB[DIM - 1][c];
+        pt[DIM - 1] += tBB * wE[DIM - 1][c];
+        V += tEE * wE[DIM - 1][c];
+      } else {
+        pt[0] = tEB;
+        pt[1] = tBE;
+        V = tEE;
+      }
+    }
+    vs[0] = V;
+#pragma unroll
+    for (int r = 0; r < DIM; r++) {
+      if ((nbmask >> lf_of<DIM>(r, cr[r])) & 1) {
+        const double diff = pt[r] - msel;
+        const double y = indicator_y(diff, msel, mI, MI);
+        double yc;
         if (g.phi == RKDG_PHI_BJ) {
           yc = y < 1.0 ? y : 1.0;
         } else if (g.phi == RKDG_PHI_VENKAT) {
@@ -1011,99 +1063,91 @@ __global__ __launch_bounds__(64) void tensor_limit_kernel(const LimitArgs A, con
           const double yRel = y / yStar;
           yc = y < 1.0 ? y + (3.0 - 2.0 * yStar) * yRel * yRel + (yStar - 2.0) * yRel * yRel * yRel : 1.0;
         }
+        yr = yc < yr ? yc : yr;
       }
-      ylane = yc < ylane ? yc : ylane;
     }
+    yr = team_min<T>(yr);
   }
-
-  // minimum over the team's lanes (min is exact, so the order does not matter)
-#pragma unroll
-  for (int off = T / 2; off > 0; off >>= 1) {
-    const double o = __shfl_xor(ylane, off, 64);
-    ylane = o < ylane ? o : ylane;
-  }
-  double yr = ylane;
   if (g.indicator == RKDG_IND_NOWHERE) yr = 1.0;
   else if (g.indicator == RKDG_IND_EVERYWHERE) yr = 0.0;
 
-  // limit: each node lane owns one node
-  const int j = lane;
-  const bool node_lane = active && lane < ND;
-  double u[NEQ];
-  if (node_lane) {
+  const bool linear = P == 1 && g.linearize && multi;
+  if constexpr (P == 1) {
+    // linearize: the multiplier and the last hope work on the element's linear
+    // reconstruction (the indicator above reads the state as it is); lane = node
+    if (linear) {
+      double lin[NEQ];
 #pragma unroll
-    for (int v = 0; v < NEQ; v++) u[v] = s_u[team][v][j];
+      for (int v = 0; v < NEQ; v++) lin[v] = linearize_q1<DIM>(ue + v * ROW, mean[v], lane);
+      __syncthreads();
+#pragma unroll
+      for (int v = 0; v < NEQ; v++) s_u[team * ES + v * ROW + lane] = lin[v];
+      __syncthreads();
+    }
   }
+
   int trouble = 0;
-  double feff = 1.0;  // the factor of the limited state mean + feff (u - mean)
-  if (g.limiter == RKDG_LIM_MULTI) {
+  double f = 1.0;  // the factor of the limited state mean + f (u - mean)
+  if (multi) {
     if (yr < 1.0) trouble = 1;
     // u <- mean + y (u - mean) applied nd times (limiter_multiplier.cpp:24-38)
     // is u <- mean + y^nd (u - mean); y^nd by repeated squaring
-    double f = yr;
+    f = yr;
     if (g.pow_nd) {
       double acc = 1.0, b = yr;
+#pragma unroll
       for (int e2 = ND; e2 > 0; e2 >>= 1) {
         if (e2 & 1) acc *= b;
         b *= b;
       }
       f = acc;
     }
-    feff = f;
-    if (node_lane) {
-#pragma unroll
-      for (int v = 0; v < NEQ; v++) u[v] = mean[v] + f * (u[v] - mean[v]);
-    }
     if (g.last_hope) {
-      bool bad_v = false;
-      // the limited state at the reference vertices: mean + f (u(vertex) - mean),
-      // u(vertex) from the two-direction partial sums (last direction here)
-      for (int it = lane; it < NVERT; it += T) {
-        if (!active) break;
-        const int cx = it & 1, cy = (it >> 1) & 1, cz = (it >> 2) & 1;
-        double vs[NEQ];
+      // the limited state at the reference vertices: mean + f (u(vertex) - mean)
 #pragma unroll
-        for (int v = 0; v < NEQ; v++) {
-          double s = 0.0;
-#pragma unroll
-          for (int b = 0; b < NB; b++) {
-            const double tt = s_ty[team][cx][cy][v][b];
-            s += DIM == 3 ? tt * tb.E[cz][b] : tt;
-          }
-          vs[v] = mean[v] + f * (s - mean[v]);
-        }
-        if (!physical<DIM>(vs, g)) bad_v = true;
+      for (int v = 0; v < NEQ; v++) {
+        if (v > 0 || !ind_bj || linear) vs[v] = at_vertex(ue + v * ROW);
+        vs[v] = mean[v] + f * (vs[v] - mean[v]);
       }
-      const unsigned long long bm = __ballot(bad_v);
-      const unsigned long long tm = T == 64 ? ~0ull : (((1ull << T) - 1ull) << (team * T));
-      if (active && (bm & tm)) {
+      const unsigned long long bm = __ballot(!physical<DIM>(vs, g));
+      if (active && ((bm >> (team * T)) & ((1ull << T) - 1ull))) {
         trouble |= 2;
-        feff = 0.0;
-        if (node_lane) {
-#pragma unroll
-          for (int v = 0; v < NEQ; v++) u[v] = mean[v];
-        }
+        f = 0.0;
       }
     }
-  } else if (g.limiter == RKDG_LIM_FINDIFF) {
+  } else if (findiff) {
     if (yr < 0.999) {
       trouble = 1;
-      feff = 0.0;
-      if (node_lane) {
+      f = 0.0;
+    }
+  }
+  if (A.troubled && active && lane == 0) A.troubled[e] = (int8_t)trouble;
+  if (A.factor) {
+    if (active && lane == 0) A.factor[e] = f;
+    return;
+  }
+  if (lane == 0) s_f[team] = f;
+  __syncthreads();
 #pragma unroll
-        for (int v = 0; v < NEQ; v++) u[v] = mean[v];
+  for (int p = 0; p < LP; p++) {
+    const int i = tid + 64 * p;
+    if (i < nn) {
+      const int el = i / ND, k = i - el * ND;
+      const double fe = s_f[el];
+      if (fe != 1.0 || linear) {
+#pragma unroll
+        for (int v = 0; v < NEQ; v++) {
+          const double m = s_mean[el][v];
+          sbase(A.x + (v * NDOFS + e0 * ND))[(unsigned)i] = m + fe * (s_u[el * ES + v * ROW + k] - m);
+        }
       }
     }
   }
-  if (A.factor) {
-    if (active && lane == 0) A.factor[e] = feff;
-  } else if (node_lane) {
-#pragma unroll
-    for (int v = 0; v < NEQ; v++) A.x[v * NDOFS + e * ND + j] = u[v];
-  }
-  if (A.troubled && active && lane == 0) A.troubled[e] = (int8_t)trouble;
 }
 
+#define RKDG_TENSOR_CASES(X) X(2, 1) X(2, 2) X(2, 3) X(2, 4) X(2, 5) X(3, 1) X(3, 2) X(3, 3)
+
+#if RKDG_TENSOR_PART == 0
 // ---------------------------------------------------------------------------
 __global__ void fill_kernel(double* p, double v, int64_t n) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -1125,7 +1169,6 @@ hipError_t launch_copy(double* dst, const double* src, int64_t n, hipStream_t s)
   return hipGetLastError();
 }
 
-#define RKDG_TENSOR_CASES(X) X(2, 1) X(2, 2) X(2, 3) X(2, 4) X(2, 5) X(3, 1) X(3, 2) X(3, 3)
 
 bool tensor_supported(int dim, int p) {
 #define X(D, PP) \
@@ -1143,6 +1186,16 @@ int tensor_elems_per_block(int dim, int p) {
   return 1;
 }
 
+#endif  // RKDG_TENSOR_PART == 0
+
+// The right-hand-side kernels are most of this file's compile time: it is built
+// as several objects, part 0 with everything else and parts 1 to 4 each with the
+// launchers of some element types (explicit instantiations at the end).
+template <int D, int PP>
+hipError_t launch_rhs_dp(const RhsArgs& a, const SchemeParams& g, const TensorTables* t,
+                         const TensorTables& th, bool bc, hipStream_t s);
+
+#if RKDG_TENSOR_PART > 0
 template <int D, int PP, int RS>
 hipError_t launch_rhs_rs(const RhsArgs& a, const SchemeParams& g, const TensorTables* t,
                          const TensorTables& th, bool bc, hipStream_t s) {
@@ -1195,6 +1248,24 @@ hipError_t launch_rhs_dp(const RhsArgs& a, const SchemeParams& g, const TensorTa
   }
 }
 
+#define RKDG_RHS_INSTANCE(D, PP)                                                                             \
+  template hipError_t launch_rhs_dp<D, PP>(const RhsArgs&, const SchemeParams&, const TensorTables*,         \
+                                           const TensorTables&, bool, hipStream_t);
+#if RKDG_TENSOR_PART == 1
+RKDG_RHS_INSTANCE(3, 1)
+#elif RKDG_TENSOR_PART == 2
+RKDG_RHS_INSTANCE(3, 2)
+#elif RKDG_TENSOR_PART == 3
+RKDG_RHS_INSTANCE(3, 3)
+#else
+RKDG_RHS_INSTANCE(2, 1)
+RKDG_RHS_INSTANCE(2, 2)
+RKDG_RHS_INSTANCE(2, 3)
+RKDG_RHS_INSTANCE(2, 4)
+RKDG_RHS_INSTANCE(2, 5)
+#endif
+#else
+
 hipError_t launch_tensor_rhs(int dim, int p, const RhsArgs& a, const SchemeParams& g,
                              const TensorTables* t, const TensorTables& th, bool has_bdr, hipStream_t s) {
 #define X(D, PP) \
@@ -1208,9 +1279,9 @@ hipError_t launch_tensor_limit(int dim, int p, const LimitArgs& a, const SchemeP
                                const TensorTables* t, hipStream_t s) {
 #define X(D, PP)                                                           \
   if (dim == D && p == PP) {                                               \
-    using C = TC<D, PP>;                                                   \
+    using C = LC<D, PP>;                                                   \
     const int64_t nb = (a.NE + C::EPB - 1) / C::EPB;                       \
-    tensor_limit_kernel<D, PP><<<(unsigned)nb, C::BLOCK, 0, s>>>(a, g, t); \
+    tensor_limit_kernel<D, PP><<<(unsigned)nb, 64, 0, s>>>(a, g, t);       \
     return hipGetLastError();                                              \
   }
   RKDG_TENSOR_CASES(X)
@@ -1222,13 +1293,15 @@ hipError_t launch_tensor_means(int dim, int p, const MeansArgs& a, const TensorT
                                hipStream_t s) {
 #define X(D, PP)                                                                      \
   if (dim == D && p == PP) {                                                          \
-    using C = TC<D, PP>;                                                              \
-    tensor_means_kernel<D, PP><<<(unsigned)((a.NE + C::EPB - 1) / C::EPB), C::BLOCK, 0, s>>>(a, t); \
+    using C = MC<D, PP>;                                                              \
+    tensor_means_kernel<D, PP><<<(unsigned)((a.NE + C::EB - 1) / C::EB), 256, 0, s>>>(a, t); \
     return hipGetLastError();                                                         \
   }
   RKDG_TENSOR_CASES(X)
 #undef X
   return hipErrorInvalidValue;
 }
+
+#endif  // RKDG_TENSOR_PART
 
 }  // namespace rkdg

@@ -6,8 +6,8 @@
 // (src/limiter/limiter.cpp:22-94, src/indicator/indicator_bj.cpp:15-200,
 // src/limiter/limiter_multiplier.cpp:12-99, src/limiter/limiter_findiff.cpp:3-33).
 //
-// Work decomposition: one team of T lanes per element (T = next power of two of
-// max(nodes, 2 * face points)); a workgroup is one 64-lane wavefront holding
+// Work decomposition: one team of T lanes per element (the next power of two of
+// max(nodes, 2 * face points), 20 for Q1 hexahedra); a workgroup is one 64-lane wavefront holding
 // EPB = 64/T elements, so every barrier is a single-wave barrier. The 1D basis
 // tables are staged in LDS, as is the element's state. The volume term is the
 // collocated weak derivative (Gauss-Legendre nodes are the volume quadrature
@@ -37,8 +37,13 @@ struct TC {
   static constexpr int NFN = DIM == 3 ? N * N : N;
   static constexpr int NVERT = DIM == 3 ? 8 : 4;
   static constexpr int NIP = DIM == 3 ? 4 : 2;  // indicator points per face (order 2 rule)
+  // lanes per element of the right-hand side. Q1 hexahedra: 20, which the 20
+  // rows of the traces and the lift and the 18 points of an axis fill, so three
+  // elements share a wavefront; 32 lanes held two of them and left 12 to 14 lanes
+  // idle in every face phase (111,813 elements, HLLC, right-hand side: 290 -> 247 us)
   static constexpr int m1 = ND > 2 * NFP ? ND : 2 * NFP;
-  static constexpr int T = m1 <= 4 ? 4 : (m1 <= 8 ? 8 : (m1 <= 16 ? 16 : (m1 <= 32 ? 32 : 64)));
+  static constexpr int T = DIM == 3 && P == 1 ? 20
+                                              : (m1 <= 4 ? 4 : (m1 <= 8 ? 8 : (m1 <= 16 ? 16 : (m1 <= 32 ? 32 : 64))));
   static constexpr int BLOCK = 64;
   static constexpr int EPB = BLOCK / T;
 };
@@ -145,8 +150,22 @@ struct TArg {
 // CV: curved (trilinear) hexahedra, role 0 only: adj(J) per node in the volume
 // term, the normal and |n| per face point, the dense inverse mass and the mass
 // weights of the means, all from the element's CurvedLayout record.
+//
+// Waves per SIMD asked of the compiler: the kernel is bound by latency as much as
+// by issue, so a wave more is worth a few spilled registers but not many. Four
+// (128 VGPRs) where that spills at most a handful, three otherwise: the rotated
+// solvers with boundary states, and those on Q1 hexahedra, whose setup phases
+// unroll further. Without a bound they took 169 to 175 VGPRs, two waves
+// (111,813 Q1 hexahedra, HLLC with walls, right-hand side: 247 us, with three 204 us);
+// four waves at 12 to 30 spills were slower than three (rotated Q2 hexahedra,
+// HLL: step 741 against 642 us), so the registers were saved first (TAB_REGS below).
+template <int DIM, int P, int RS, bool BC, bool CV>
+constexpr int rhs_waves() {
+  if ((CV && (P == 3 || RS == RKDG_RS_HLLC)) || (DIM == 2 && P == 5)) return 3;
+  return RS == RKDG_RS_RUSANOV || (!BC && P >= 2) ? 4 : 3;
+}
 template <int DIM, int P, int RS, bool BC, int ROLE, bool AL, bool CV = false>
-__global__ __launch_bounds__(64, ROLE == 1 ? 4 : 1) void tensor_rhs_kernel(const RhsArgs A, const SchemeParams g,
+__global__ __launch_bounds__(64, (ROLE == 1 ? 4 : rhs_waves<DIM, P, RS, BC, CV>())) void tensor_rhs_kernel(const RhsArgs A, const SchemeParams g,
                                                         const TensorTables* __restrict__ gtb,
                                                         const TArg<DIM, P + 1, TC<DIM, P>::NQ> ka) {
   const TT<P + 1, TC<DIM, P>::NQ>& kt = ka.t;
@@ -197,7 +216,7 @@ __global__ __launch_bounds__(64, ROLE == 1 ? 4 : 1) void tensor_rhs_kernel(const
   const int64_t e0 = blk * EPB;  // ROLE 0: the block's first element
   const int64_t li = blk0 * EPB + team;  // ROLES 1, 2: this team's index in the element list
   const int64_t e = ROLE == 0 ? e0 + team : (li < A.nlist ? (int64_t)A.elist[li] : (int64_t)0);
-  const bool active = ROLE == 0 ? e < NE : li < A.nlist;
+  const bool active = team < EPB && (ROLE == 0 ? e < NE : li < A.nlist);
 
   // ---- phase 0: tables, element state, connectivity, normals and geometry
   // into LDS. Every load is issued before the first LDS store: one memory round
@@ -371,15 +390,22 @@ __global__ __launch_bounds__(64, ROLE == 1 ? 4 : 1) void tensor_rhs_kernel(const
     // ---- face terms, one axis at a time. Phases per axis r: points(r) |
     // lift(r) + traces(r+1) | node accumulation(r) + points(r+1) ..., so each
     // axis costs two barriers.
-    // Table values that depend on the lane but not on the axis, read from LDS
-    // once (the phases below are one pass of the team when ONE_PASS; otherwise
-    // they read the tables per item).
+    // Table values that depend on the lane but not on the axis: kept in registers
+    // over the axes (the phases below are one pass of the team when ONE_PASS)
+    // where they fit the registers of the waves asked for: at three waves, and in
+    // the aligned interior Rusanov form on Q2 hexahedra at four. The others read
+    // them from LDS again in each phase, 12 to 26 VGPRs less, which is what lets
+    // the rotated solvers on Q2 and Q3 hexahedra and the curved Rusanov form run
+    // at four (63,360 rotated Q2 hexahedra, HLL: step 642 -> 601 us; 29,760 curved
+    // ones, Rusanov: 481 -> 436 us; 29,667 Q3 hexahedra, LLF: 643 -> 624 us)
     constexpr bool ONE_PASS = 2 * NEQ * N <= T && 2 * NFP <= T;
+    constexpr bool TAB_REGS = ONE_PASS && ((ROLE == 0 && rhs_waves<DIM, P, RS, BC, CV>() == 3) ||
+                                           (AL && !BC && DIM == 3 && P == 2 && RS == RKDG_RS_RUSANOV));
     double ec[N];         // traces: E[c][k] of the lane's face side
     double bqj[N];        // points: B[qj][b] of the lane's point
     double bqa[NQ];       // lift: B[qi][a] of the lane's row
     double wq2 = 0.0;     // points: the lane's face weight
-    if (ONE_PASS) {
+    if (TAB_REGS) {
       const int ct = lane / (NEQ * NB);
       const int at = (lane - (lane / (NEQ * N)) * (NEQ * N)) % N;
       const int qt = lane % NFP, qit = qt % NQ, qjt = DIM == 3 ? qt / NQ : 0;
@@ -429,7 +455,7 @@ __global__ __launch_bounds__(64, ROLE == 1 ? 4 : 1) void tensor_rhs_kernel(const
         for (int a = 0; a < N; a++) {
           double t = 0.0;
   #pragma unroll
-          for (int k = 0; k < N; k++) t += s_u[team][v][vnode<DIM, N>(r, k, a, b)] * (ONE_PASS ? ec[k] : tb.E[c][k]);
+          for (int k = 0; k < N; k++) t += s_u[team][v][vnode<DIM, N>(r, k, a, b)] * (TAB_REGS ? ec[k] : tb.E[c][k]);
           tr[a] = t;
         }
   #pragma unroll
@@ -476,7 +502,7 @@ __global__ __launch_bounds__(64, ROLE == 1 ? 4 : 1) void tensor_rhs_kernel(const
           double t = 0.0;
           if (DIM == 3) {
   #pragma unroll
-            for (int b = 0; b < N; b++) t += s_to[team][c][v][qi][b] * (ONE_PASS ? bqj[b] : tb.B[qj][b]);
+            for (int b = 0; b < N; b++) t += s_to[team][c][v][qi][b] * (TAB_REGS ? bqj[b] : tb.B[qj][b]);
           } else {
             t = s_to[team][c][v][qi][0];
           }
@@ -515,7 +541,7 @@ __global__ __launch_bounds__(64, ROLE == 1 ? 4 : 1) void tensor_rhs_kernel(const
             double t = 0.0;
             if (DIM == 3) {
   #pragma unroll
-              for (int b = 0; b < N; b++) t += s_tn[team][c][v][pi][b] * ((AL && ONE_PASS) ? bqj[b] : tb.B[pj][b]);
+              for (int b = 0; b < N; b++) t += s_tn[team][c][v][pi][b] * ((AL && TAB_REGS) ? bqj[b] : tb.B[pj][b]);
             } else {
               t = s_tn[team][c][v][pi][0];
             }
@@ -543,7 +569,7 @@ __global__ __launch_bounds__(64, ROLE == 1 ? 4 : 1) void tensor_rhs_kernel(const
         }
         if (!ok || lam < 0.0) atomicMin(&s_bad[team], f);  // classified and reported at the end
         else lmax = lam > lmax ? lam : lmax;
-        const double wgt = (ONE_PASS ? wq2 : (DIM == 3 ? tb.wq[qi] * tb.wq[qj] : tb.wq[qi])) * snm;  // flux sign * w_q * |n|
+        const double wgt = (TAB_REGS ? wq2 : (DIM == 3 ? tb.wq[qi] * tb.wq[qj] : tb.wq[qi])) * snm;  // flux sign * w_q * |n|
   #pragma unroll
         for (int v = 0; v < NEQ; v++) work[(c * NEQ + v) * RW + q] = fl[v] * wgt;
       }
@@ -561,7 +587,7 @@ __global__ __launch_bounds__(64, ROLE == 1 ? 4 : 1) void tensor_rhs_kernel(const
           for (int qj = 0; qj < NQ; qj++) {
             double tt = 0.0;
   #pragma unroll
-            for (int qi = 0; qi < NQ; qi++) tt += w[qi + NQ * qj] * (ONE_PASS ? bqa[qi] : tb.B[qi][a]);
+            for (int qi = 0; qi < NQ; qi++) tt += w[qi + NQ * qj] * (TAB_REGS ? bqa[qi] : tb.B[qi][a]);
             W[qj] = tt;
           }
   #pragma unroll

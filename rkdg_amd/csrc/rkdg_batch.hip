@@ -25,7 +25,7 @@ __global__ __launch_bounds__(256) void batch_init_kernel(BatchTime b) {
   __syncthreads();
   int n = 0;
   for (int i = threadIdx.x; i < b.count; i += blockDim.x) {
-    b.dt[i] = next_dt(b.cfl, b.hmin[i], b.lam[i], b.p);
+    b.dt[i] = next_dt(b.cfl, b.hmin[i], take_lambda(b.lam, b.lam_ld, i), b.p);
     b.dt_real[i] = b.dt[i];
     b.steps[i] = 0;
     b.active[i] = 1;
@@ -55,7 +55,7 @@ __global__ __launch_bounds__(256) void batch_post_kernel(BatchTime b) {
   int n = 0;
   for (int i = threadIdx.x; i < b.count; i += blockDim.x) {
     if (!b.active[i]) continue;
-    const double dt = next_dt(b.cfl, b.hmin[i], b.lam[i], b.p);
+    const double dt = next_dt(b.cfl, b.hmin[i], take_lambda(b.lam, b.lam_ld, i), b.p);
     const double t = b.t[i] + dt;
     b.dt[i] = dt;
     b.t[i] = t;
@@ -70,7 +70,21 @@ __global__ __launch_bounds__(256) void batch_post_kernel(BatchTime b) {
   if (threadIdx.x == 0) b.n_active[0] = s_n;
 }
 
+__global__ __launch_bounds__(256) void batch_status_kernel(BatchTime b, double* out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= b.count) return;
+  out[i] = b.t[i];
+  out[b.count + i] = b.dt[i];
+  out[2 * b.count + i] = (double)b.steps[i];
+  out[3 * b.count + i] = (double)b.active[i];
+}
+
 }  // namespace
+
+hipError_t launch_batch_status(const BatchTime& b, double* out, hipStream_t s) {
+  batch_status_kernel<<<(b.count + 255) / 256, 256, 0, s>>>(b, out);
+  return hipGetLastError();
+}
 
 hipError_t launch_batch_init(const BatchTime& b, hipStream_t s) {
   batch_init_kernel<<<1, 256, 0, s>>>(b);

@@ -436,9 +436,9 @@ __device__ __forceinline__ void dense_rhs_block(const RhsArgs& A, const SchemePa
         const double o = __shfl_xor(lmax, off, 64);
         lmax = o > lmax ? o : lmax;
       }
-      if (tid == 0) atomic_max_pos(A.lam + i0, lmax);
+      if (tid == 0) atomic_max_pos(lam_slot(A.lam, A.lam_ld) + i0, lmax);
     } else if (active) {
-      atomic_max_pos(A.lam + ins, lmax);
+      atomic_max_pos(lam_slot(A.lam, A.lam_ld) + ins, lmax);
     }
   }
   __syncthreads();  // LDS is reused by the next work block

@@ -149,7 +149,8 @@ struct rkdg_ctx {
   double* d_geo = nullptr;
   int* d_nbr = nullptr;
   int* d_fcode = nullptr;
-  double* d_lam = nullptr;    // per-stage wave speeds [8]
+  double* d_lam = nullptr;    // wave speeds [kLamSlots][lam_stride(count)], zero between uses
+  bool lam_dirty = false;     // a launch that adds to d_lam was enqueued and nothing has taken it yet
   long long* d_err = nullptr;
   int64_t err_pair[2] = {-1, -1};  // element pair of the last reported device error
   double* d_means = nullptr;
@@ -157,7 +158,9 @@ struct rkdg_ctx {
   // factors of the steps that apply the limiter on load
   double* d_means2 = nullptr;
   double* d_fac = nullptr;
-  long long* h_pin = nullptr;    // pinned host words: device error word [4], then the wave speeds [count]
+  // pinned host words: device error word [4], active instances, then the wave speeds [count] and the
+  // batch status [4][count]
+  long long* h_pin = nullptr;
   int* d_order = nullptr;        // tensor contexts: work blocks in Morton order of their centroids
   // two-coloured tensor meshes (bipartite face graph, no boundary faces): the
   // solver and receiver element lists (each in Morton order of the element
@@ -772,8 +775,8 @@ int build_dense(rkdg_ctx* c, const rkdg_mesh_desc* m) {
   HIP_TRY(hipMemcpy(c->d_dtab, tab.data(), sizeof(double) * tsize, hipMemcpyHostToDevice));
   HIP_TRY(hipMalloc(&c->d_rtab, sizeof(double) * rtab.size()));
   HIP_TRY(hipMemcpy(c->d_rtab, rtab.data(), sizeof(double) * rtab.size(), hipMemcpyHostToDevice));
-  HIP_TRY(hipMalloc(&c->d_lam, sizeof(double) * 8 * c->count));
-  HIP_TRY(hipMemset(c->d_lam, 0, sizeof(double) * 8 * c->count));
+  HIP_TRY(hipMalloc(&c->d_lam, sizeof(double) * kLamSlots * lam_stride(c->count)));
+  HIP_TRY(hipMemset(c->d_lam, 0, sizeof(double) * kLamSlots * lam_stride(c->count)));
   HIP_TRY(hipMalloc(&c->d_err, sizeof(long long) * 4));
   HIP_TRY(hipMemset(c->d_err, 0, sizeof(long long) * 4));
   HIP_TRY(hipMalloc(&c->d_means, sizeof(double) * c->neq * NE));
@@ -1505,8 +1508,8 @@ int build_ctx(rkdg_ctx* c, const rkdg_mesh_desc* m, const rkdg_scheme_desc* s) {
   c->nbr_h = nbr;
   HIP_TRY(hipMalloc(&c->d_fcode, sizeof(int) * nf * NE));
   HIP_TRY(hipMemcpy(c->d_fcode, fcode.data(), sizeof(int) * nf * NE, hipMemcpyHostToDevice));
-  HIP_TRY(hipMalloc(&c->d_lam, sizeof(double) * 8 * c->count));
-  HIP_TRY(hipMemset(c->d_lam, 0, sizeof(double) * 8 * c->count));
+  HIP_TRY(hipMalloc(&c->d_lam, sizeof(double) * kLamSlots * lam_stride(c->count)));
+  HIP_TRY(hipMemset(c->d_lam, 0, sizeof(double) * kLamSlots * lam_stride(c->count)));
   HIP_TRY(hipMalloc(&c->d_err, sizeof(long long) * 4));
   HIP_TRY(hipMemset(c->d_err, 0, sizeof(long long) * 4));
   HIP_TRY(hipMalloc(&c->d_means, sizeof(double) * c->neq * NE));
@@ -1632,8 +1635,9 @@ hipError_t rhs_launch(rkdg_ctx* c, const RhsArgs& a0) {
       na.geo = c->d_ncgeo;
       na.out = c->d_ncbuf;
       na.lam = a.lam;
+      na.lam_ld = a.lam_ld;
       na.err = a.err;
-      na.no_lambda = a.no_lambda && !a.face_only;
+      na.no_lambda = a.no_lambda;
       e = launch_nc_faces(c->dim, c->p, na, c->sp, c->d_tb, c->stream);
       a.ncslot = c->d_ncslot;
       a.ncbuf = c->d_ncbuf;
@@ -1657,6 +1661,8 @@ RhsArgs base_args(rkdg_ctx* c, const double* x) {
   a.fcode = c->d_fcode;
   a.NE = c->NE;
   a.lam = c->d_lam;
+  a.lam_ld = lam_stride(c->count);
+  a.no_lambda = 1;  // want_lambda() where it is read
   a.err = c->d_err;
   a.face_only = 0;
   a.inst = c->d_inst;
@@ -1668,19 +1674,28 @@ RhsArgs base_args(rkdg_ctx* c, const double* x) {
   return a;
 }
 
-// pinned host words for the per-step readbacks (a copy to pageable memory is
-// staged by the runtime and costs tens of microseconds per step)
+// pinned host words for the per-step readbacks, which a kernel writes
+// (launch_publish)
+constexpr int kPinWords = 8;  // ahead of the wave speeds
 hipError_t ensure_pinned(rkdg_ctx* c) {
   if (c->h_pin) return hipSuccess;
-  return hipHostMalloc(reinterpret_cast<void**>(&c->h_pin), sizeof(long long) * 4 + sizeof(double) * c->count,
+  return hipHostMalloc(reinterpret_cast<void**>(&c->h_pin), sizeof(long long) * (kPinWords + 5 * (size_t)c->count),
                        hipHostMallocDefault);
 }
+double* pinned_lambda(rkdg_ctx* c) { return reinterpret_cast<double*>(c->h_pin + kPinWords); }
 
-int check_device_error(rkdg_ctx* c, int64_t* info) {
-  HIP_TRY(ensure_pinned(c));
-  long long* h = c->h_pin;
-  HIP_TRY(hipMemcpyAsync(h, c->d_err, sizeof(long long) * 4, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
+// the launch of `a` adds its wave speeds to d_lam
+int want_lambda(rkdg_ctx* c, RhsArgs& a) {
+  if (c->lam_dirty)  // an earlier call failed between its launch and its reading
+    HIP_TRY(launch_fill(c->d_lam, 0.0, (int64_t)kLamSlots * a.lam_ld, c->stream));
+  c->lam_dirty = true;
+  a.no_lambda = 0;
+  return RKDG_OK;
+}
+
+// the error word as published to the pinned words (the stream is synchronized)
+int report_device_error(rkdg_ctx* c, int64_t* info) {
+  const long long* h = c->h_pin;
   if (h[0]) {
     const long long kind = h[0], e1 = h[1], e2 = h[2];
     c->err_pair[0] = e1;
@@ -1700,13 +1715,30 @@ int check_device_error(rkdg_ctx* c, int64_t* info) {
   return RKDG_OK;
 }
 
-// wave speed of stage slot; on a batch, the maximum over the instances
-int read_lambda(rkdg_ctx* c, int slot, double* lam) {
+// Publishes the error word (and, where asked, the wave speeds and the number of
+// active instances), synchronizes and reports a device error.
+int check_device_error(rkdg_ctx* c, int64_t* info, bool lambda = false, bool active = false) {
   HIP_TRY(ensure_pinned(c));
-  double* h = reinterpret_cast<double*>(c->h_pin + 4);
-  HIP_TRY(hipMemcpyAsync(h, c->d_lam + (int64_t)slot * c->count, sizeof(double) * c->count,
-                         hipMemcpyDeviceToHost, c->stream));
-  const int rc = check_device_error(c, nullptr);
+  PublishArgs p{};
+  p.count = c->count;
+  p.lam_ld = lam_stride(c->count);
+  if (lambda) p.lam = c->d_lam;
+  p.lam_out = pinned_lambda(c);
+  p.err = c->d_err;
+  p.err_out = c->h_pin;
+  if (active) p.n_active = c->d_nact;
+  p.n_active_out = c->h_pin + 4;
+  HIP_TRY(launch_publish(p, c->stream));
+  if (lambda) c->lam_dirty = false;
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  return report_device_error(c, info);
+}
+
+// wave speed of the launch that asked for it; on a batch, the maximum over the instances
+int read_lambda(rkdg_ctx* c, double* lam) {
+  const int rc = check_device_error(c, nullptr, true);
+  if (rc == RKDG_E_HIP) return rc;
+  const double* h = pinned_lambda(c);
   *lam = *std::max_element(h, h + c->count);
   return rc;
 }
@@ -1777,7 +1809,7 @@ bool is_ssprk3(int s, const double* a, const double* b) {
 // stage input come out of the same epilogue for the limiter. buf[0..s-2] hold
 // W_1..W_{s-1}, buf[3] the accumulator; every one is written before it is read
 // (stage 0 has no bases), so nothing needs clearing. The last stage's wave
-// speed lands in d_lam[s-1] when want_lambda.
+// speed goes to d_lam when with_lambda.
 //
 // Where limit_on_load holds, the limiter of a stage input W_i is a factor pass
 // (it writes one factor per element, not W_i) and the stage kernel limits W_i
@@ -1790,20 +1822,21 @@ bool is_ssprk3(int s, const double* a, const double* b) {
 // The means alternate between two buffers (a stage reads the means of its
 // input while it writes those of its output); the last stage's are in d_means.
 int step_impl(rkdg_ctx* c, double* x, double dt, int s, const double* a, const double* b, double* const* buf,
-              bool want_lambda) {
+              bool with_lambda) {
   double* W[4] = {nullptr, buf[0], buf[1], buf[2]};
   double* acc = buf[3];
   const bool onload = limit_on_load(c);
   const bool so = onload && is_ssprk3(s, a, b);
-  HIP_TRY(launch_fill(c->d_lam, 0.0, 8 * c->count, c->stream));
   auto A_ = [&](int i, int j) { return a[i * (i - 1) / 2 + j]; };
   auto mbuf = [&](int i) { return (!onload || (s - 1 - i) % 2 == 0) ? c->d_means : c->d_means2; };
   for (int i = 0; i < s; i++) {
     const double* in = i == 0 ? x : W[i];
     RhsArgs ra = base_args(c, in);
-    ra.lam = c->d_lam + (int64_t)i * c->count;
     const bool last = i == s - 1;
-    ra.no_lambda = (!last || !want_lambda) ? 1 : 0;  // only the last stage's wave speed is read
+    if (last && with_lambda) {  // only the last stage's wave speed is read
+      const int rc = want_lambda(c, ra);
+      if (rc) return rc;
+    }
     if (onload && i > 0) {
       ra.lim_f = c->d_fac;
       ra.lim_mean = mbuf(i - 1);
@@ -1841,7 +1874,7 @@ int step_impl(rkdg_ctx* c, double* x, double dt, int s, const double* a, const d
   return RKDG_OK;
 }
 
-BatchTime batch_time(rkdg_ctx* c, const double* lam) {
+BatchTime batch_time(rkdg_ctx* c) {
   BatchTime b{};
   b.count = c->count;
   b.t = c->d_t;
@@ -1849,7 +1882,8 @@ BatchTime batch_time(rkdg_ctx* c, const double* lam) {
   b.dt_real = c->d_dtr;
   b.t_final = c->d_tf;
   b.hmin = c->d_hmin;
-  b.lam = lam;
+  b.lam = c->d_lam;
+  b.lam_ld = lam_stride(c->count);
   b.active = c->d_active;
   b.steps = c->d_steps;
   b.n_active = c->d_nact;
@@ -1864,15 +1898,16 @@ BatchTime batch_time(rkdg_ctx* c, const double* lam) {
 int batch_step_launch(rkdg_ctx* c, double* x, int s, const double* a, const double* b) {
   double* W[4] = {nullptr, c->d_stage[0], c->d_stage[1], c->d_stage[2]};
   double* acc = c->d_stage[3];
-  HIP_TRY(launch_fill(c->d_lam, 0.0, (int64_t)s * c->count, c->stream));
-  BatchTime bt = batch_time(c, c->d_lam + (int64_t)(s - 1) * c->count);
+  BatchTime bt = batch_time(c);
   HIP_TRY(launch_batch_pre(bt, c->stream));
   auto A_ = [&](int i, int j) { return a[i * (i - 1) / 2 + j]; };
   for (int i = 0; i < s; i++) {
     const double* in = i == 0 ? x : W[i];
     RhsArgs ra = base_args(c, in);
-    ra.lam = c->d_lam + (int64_t)i * c->count;
-    ra.no_lambda = i < s - 1 ? 1 : 0;  // only the last stage's wave speeds are read
+    if (i == s - 1) {  // only the last stage's wave speeds are read
+      const int rc = want_lambda(c, ra);
+      if (rc) return rc;
+    }
     ra.dt_inst = c->d_dtr;
     ra.active = c->d_active;
     int n = 0;
@@ -1895,6 +1930,7 @@ int batch_step_launch(rkdg_ctx* c, double* x, int s, const double* a, const doub
     if (rc) return rc;
   }
   HIP_TRY(launch_batch_post(bt, c->stream));
+  c->lam_dirty = false;
   return RKDG_OK;
 }
 
@@ -1995,11 +2031,9 @@ int ensure_records(rkdg_ctx* c, int s, int64_t steps) {
 // forward step from r.x recording the stage states; the limited output goes to xout
 int step_record(rkdg_ctx* c, const StepRec& r, double* xout, double dt, int s, const double* a, const double* b) {
   auto A_ = [&](int i, int j) { return a[i * (i - 1) / 2 + j]; };
-  HIP_TRY(launch_fill(c->d_lam, 0.0, 8 * c->count, c->stream));
   for (int i = 0; i < s; i++) {
     const double* in = i == 0 ? r.x : r.w[i - 1];
     RhsArgs ra = base_args(c, in);
-    ra.lam = c->d_lam + (int64_t)i * c->count;
     int n = 0;
     for (int j = i + 1; j < s; j++) {
       ra.outs[n].out = r.v[j - 1];
@@ -2374,21 +2408,24 @@ int rkdg_set_stream(rkdg_ctx* c, void* stream) {
 
 int rkdg_rhs(rkdg_ctx* c, const double* x, double* y, double* lambda_max) {
   if (!c || !x || !y) return fail(RKDG_E_ARG, "null argument");
-  HIP_TRY(launch_fill(c->d_lam, 0.0, c->count, c->stream));
   RhsArgs a = base_args(c, x);
   a.k = y;
+  if (lambda_max) {
+    const int rc = want_lambda(c, a);
+    if (rc) return rc;
+  }
   HIP_TRY(rhs_launch(c, a));
-  if (lambda_max) return read_lambda(c, 0, lambda_max);
-  return RKDG_OK;
+  return lambda_max ? read_lambda(c, lambda_max) : RKDG_OK;
 }
 
 int rkdg_face_lambda(rkdg_ctx* c, const double* x, double* lambda_max) {
   if (!c || !x || !lambda_max) return fail(RKDG_E_ARG, "null argument");
-  HIP_TRY(launch_fill(c->d_lam, 0.0, c->count, c->stream));
   RhsArgs a = base_args(c, x);
   a.face_only = 1;
+  const int rc = want_lambda(c, a);
+  if (rc) return rc;
   HIP_TRY(rhs_launch(c, a));
-  return read_lambda(c, 0, lambda_max);
+  return read_lambda(c, lambda_max);
 }
 
 int rkdg_limit(rkdg_ctx* c, double* x, int8_t* troubled) {
@@ -2416,7 +2453,7 @@ int rkdg_step(rkdg_ctx* c, double* x, double t, double dt, int s, const double* 
   if (rc) return rc;
   rc = step_impl(c, x, dt, s, a, b, c->d_stage, lambda_max != nullptr);
   if (rc) return rc;
-  if (lambda_max) return read_lambda(c, s - 1, lambda_max);
+  if (lambda_max) return read_lambda(c, lambda_max);
   return RKDG_OK;
 }
 
@@ -2433,14 +2470,15 @@ int rkdg_step_ssprk3(rkdg_ctx* c, double* x, double t, double dt, double* lambda
   int rc = ensure_stage_buffers(c, 2);
   if (rc) return rc;
   double* U[2] = {c->d_stage[0], c->d_stage[1]};
-  HIP_TRY(launch_fill(c->d_lam, 0.0, 8 * c->count, c->stream));
   const double wb[3] = {0.0, 0.75, 1.0 / 3.0}, wi[3] = {0.0, 0.25, 2.0 / 3.0};
   for (int i = 0; i < 3; i++) {
     const double* in = i == 0 ? x : U[i - 1];
     double* out = i == 2 ? x : U[i];
     RhsArgs ra = base_args(c, in);
-    ra.lam = c->d_lam + (int64_t)i * c->count;
-    ra.no_lambda = (i < 2 || !lambda_max) ? 1 : 0;
+    if (i == 2 && lambda_max) {
+      rc = want_lambda(c, ra);
+      if (rc) return rc;
+    }
     ra.nout = 1;
     ra.outs[0].out = out;
     ra.outs[0].base = i == 0 ? nullptr : x;
@@ -2453,7 +2491,7 @@ int rkdg_step_ssprk3(rkdg_ctx* c, double* x, double t, double dt, double* lambda
     rc = limit_impl(c, out, nullptr, true);
     if (rc) return rc;
   }
-  if (lambda_max) return read_lambda(c, 2, lambda_max);
+  if (lambda_max) return read_lambda(c, lambda_max);
   return RKDG_OK;
 }
 
@@ -2480,7 +2518,15 @@ int rkdg_step_noalloc(rkdg_ctx* c, double* x, double t, double dt, int s, const 
   for (int i = 0; i < 4; i++) W[i] = c->scratch + i * sz;
   int rc = step_impl(c, x, dt, s, a, b, W, lambda_dev != nullptr);
   if (rc) return rc;
-  if (lambda_dev) HIP_TRY(launch_copy(lambda_dev, c->d_lam + (int64_t)(s - 1) * c->count, 1, c->stream));
+  if (lambda_dev) {
+    PublishArgs p{};
+    p.lam = c->d_lam;
+    p.lam_ld = lam_stride(c->count);
+    p.count = 1;
+    p.lam_out = lambda_dev;
+    HIP_TRY(launch_publish(p, c->stream));
+    c->lam_dirty = c->count > 1;  // a batch context: the other instances' words are still set
+  }
   return RKDG_OK;
 }
 
@@ -2976,12 +3022,13 @@ int rkdg_batch_init(rkdg_ctx* c, double* x, const double* t0, const double* t_fi
   HIP_TRY(hipMemcpyAsync(c->d_t, t0, sizeof(double) * c->count, hipMemcpyHostToDevice, c->stream));
   int rc = limit_impl(c, x, nullptr, false);
   if (rc) return rc;
-  HIP_TRY(launch_fill(c->d_lam, 0.0, c->count, c->stream));
   RhsArgs a = base_args(c, x);
   a.face_only = 1;
+  rc = want_lambda(c, a);
+  if (rc) return rc;
   HIP_TRY(rhs_launch(c, a));
-  BatchTime b = batch_time(c, c->d_lam);
-  HIP_TRY(launch_batch_init(b, c->stream));
+  HIP_TRY(launch_batch_init(batch_time(c), c->stream));
+  c->lam_dirty = false;
   return check_device_error(c, nullptr);
 }
 
@@ -3032,10 +3079,8 @@ int rkdg_batch_advance(rkdg_ctx* c, double* x, int s, const double* a, const dou
       if (rc) return rc;
     }
   }
-  int h = 0;
-  HIP_TRY(hipMemcpyAsync(&h, c->d_nact, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  rc = check_device_error(c, nullptr);
-  if (n_active) *n_active = h;
+  rc = check_device_error(c, nullptr, false, true);
+  if (n_active && rc != RKDG_E_HIP) *n_active = (int)c->h_pin[4];
   return rc;
 }
 
@@ -3044,15 +3089,16 @@ int rkdg_batch_status(rkdg_ctx* c, double* t, double* dt, int64_t* steps, int* a
   if (!c) return fail(RKDG_E_ARG, "null context");
   if (!c->d_inst) return fail(RKDG_E_ARG, "not a batch context");
   const size_t n = c->count;
+  HIP_TRY(ensure_pinned(c));
+  double* h = pinned_lambda(c) + n;
+  HIP_TRY(launch_batch_status(batch_time(c), h, c->bstream));
   HIP_TRY(hipStreamSynchronize(c->bstream));
-  if (t) HIP_TRY(hipMemcpy(t, c->d_t, sizeof(double) * n, hipMemcpyDeviceToHost));
-  if (dt) HIP_TRY(hipMemcpy(dt, c->d_dt, sizeof(double) * n, hipMemcpyDeviceToHost));
-  if (steps) {
-    std::vector<long long> h(n);
-    HIP_TRY(hipMemcpy(h.data(), c->d_steps, sizeof(long long) * n, hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < n; i++) steps[i] = h[i];
+  for (size_t i = 0; i < n; i++) {
+    if (t) t[i] = h[i];
+    if (dt) dt[i] = h[n + i];
+    if (steps) steps[i] = (int64_t)h[2 * n + i];
+    if (active) active[i] = (int)h[3 * n + i];
   }
-  if (active) HIP_TRY(hipMemcpy(active, c->d_active, sizeof(int) * n, hipMemcpyDeviceToHost));
   return RKDG_OK;
 }
 

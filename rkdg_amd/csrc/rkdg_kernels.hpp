@@ -47,19 +47,19 @@ struct RhsArgs {
   const int* nbr;      // [lf][NE] neighbour element, or -1-bc_slot for boundary faces
   const int* fcode;    // [lf][NE] bits 0-2 neighbour local face, 3-5 orientation, 6 = Elem1
   int64_t NE;
-  double* lam;         // device max wave speed (non-negative doubles compared as int64)
+  double* lam;         // wave speeds: kLamSlots rows of lam_ld, one entry per instance (lam_slot)
+  int lam_ld;
   long long* err;      // device error word [4]: flag, e1, e2, local face
   int face_only;       // first-dt path: face terms and wave speeds only, no outputs
   // batched ensembles (all null for a single instance): element -> instance,
   // per-instance step size multiplying every stage coefficient, per-instance
-  // boundary parameters [inst][RKDG_MAX_BC][8], per-instance active flag; lam
-  // then holds one slot per instance
+  // boundary parameters [inst][RKDG_MAX_BC][8], per-instance active flag
   const int* inst;
   const double* dt_inst;
   const double* bcp;
   const int* active;
   int grid_cap;  // dense kernel: persistent grid of at most this many workgroups (0: one per work block)
-  int no_lambda; // 1: the wave speed of this launch is not needed (tensor kernel skips the nodal one)
+  int no_lambda; // 1: the wave speed of this launch is not needed
   // tensor kernel (nullable): work block processed by each workgroup (a block is
   // the EPB elements from block * EPB), in an order that keeps face neighbours
   // close in time so their gathered states are still in L2
@@ -211,6 +211,29 @@ struct StateRegs {
   }
 };
 
+// The wave speed of a launch is a maximum over all its waves. One word for all
+// of them is a queue at one memory channel, in the read that comes before the
+// atomic as in the atomic itself: 59,000 waves took 120 us longer with the wave
+// speed than without (HLL on 473,000 Q1 quadrilaterals: 313 and 190 us), and 2016
+// waves 20 us. The waves are spread over kLamSlots words, each row of
+// them on a 128-byte line of its own, and the reader takes the maximum of the rows
+// and clears them for the next launch (launch_publish, take_lambda).
+constexpr int kLamSlots = 64;
+__host__ __device__ __forceinline__ int lam_stride(int count) { return (count + 15) / 16 * 16; }
+__device__ __forceinline__ double* lam_slot(double* lam, int ld) {
+  return lam + (int64_t)(blockIdx.x % kLamSlots) * ld;
+}
+__device__ __forceinline__ double take_lambda(double* lam, int ld, int i) {
+  double m = 0.0;
+#pragma unroll 16
+  for (int s = 0; s < kLamSlots; s++) {
+    const double v = lam[(int64_t)s * ld + i];
+    m = v > m ? v : m;
+  }
+  for (int s = 0; s < kLamSlots; s++) lam[(int64_t)s * ld + i] = 0.0;
+  return m;
+}
+
 // Max-accumulate a non-negative double into *addr (non-negative doubles order
 // like their bit patterns). The current value is read first and only a larger
 // value issues the atomic: one same-address atomic per workgroup over a whole
@@ -286,6 +309,20 @@ hipError_t launch_tensor_limit(int dim, int p, const LimitArgs& a, const SchemeP
 hipError_t launch_tensor_means(int dim, int p, const MeansArgs& a, const TensorTables* t,
                                hipStream_t s);
 hipError_t launch_fill(double* p, double v, int64_t n, hipStream_t s);
+// what a host call reads back, written by one kernel (in place of a copy for each,
+// which the stream runs one after the other at about 10 us apiece): the wave
+// speed of every instance (cleared for the next launch), the error word and the
+// number of active instances; each source nullable
+struct PublishArgs {
+  double* lam;
+  int lam_ld, count;
+  double* lam_out;
+  const long long* err;
+  long long* err_out;
+  const int* n_active;
+  long long* n_active_out;
+};
+hipError_t launch_publish(const PublishArgs& a, hipStream_t s);
 // diagnostics (rkdg_io.hip): partial[b*neq + v] over nblocks fixed element
 // ranges; primitive fields (and their weighted accumulation); evaluation at
 // reference points with a basis table phi[npts][nd]
@@ -323,7 +360,8 @@ struct NcArgs {
   const double* geo;      // [records][NP][3 DIM + 1]: per point the slave and master reference
                           // coordinates, weight * |n| and the slave's outward unit normal
   double* out;            // [n_elem][NEQ][ND]
-  double* lam;            // wave speed slot
+  double* lam;            // wave speeds (RhsArgs::lam)
+  int lam_ld;
   long long* err;
   int no_lambda;
 };
@@ -414,7 +452,8 @@ struct BatchTime {
   double* dt_real;      // size of the step being taken: min(dt, t_final - t)
   const double* t_final;
   const double* hmin;
-  const double* lam;    // wave-speed slot of each instance (first dt: face speeds; after a step: last stage)
+  double* lam;          // wave speeds (first dt: face speeds; after a step: last stage), taken and cleared
+  int lam_ld;
   int* active;
   long long* steps;
   int* n_active;        // [1]
@@ -425,5 +464,7 @@ struct BatchTime {
 hipError_t launch_batch_init(const BatchTime& b, hipStream_t s);  // t holds the start times
 hipError_t launch_batch_pre(const BatchTime& b, hipStream_t s);
 hipError_t launch_batch_post(const BatchTime& b, hipStream_t s);
+// t, dt, steps and active of every instance to out[4][count]
+hipError_t launch_batch_status(const BatchTime& b, double* out, hipStream_t s);
 
 }  // namespace rkdg

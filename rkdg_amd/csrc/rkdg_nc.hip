@@ -207,7 +207,7 @@ __global__ __launch_bounds__(256) void nc_face_kernel(const NcArgs A, const Sche
       const double o = __shfl_xor(lmax, off, 64);
       lmax = o > lmax ? o : lmax;
     }
-    if (tid == 0) atomic_max_pos(A.lam, lmax);
+    if (tid == 0) atomic_max_pos(lam_slot(A.lam, A.lam_ld), lmax);
   }
 }
 

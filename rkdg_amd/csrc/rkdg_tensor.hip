@@ -775,7 +775,7 @@ __global__ __launch_bounds__(64, (ROLE == 1 ? 4 : rhs_waves<DIM, P, RS, BC, CV>(
       const double o = __shfl_xor(lmax, off, 64);
       lmax = o > lmax ? o : lmax;
     }
-    if (tid == 0) atomic_max_pos(A.lam, lmax);
+    if (tid == 0) atomic_max_pos(lam_slot(A.lam, A.lam_ld), lmax);
   }
 
   // ---- a failed flux: the element pair, and whether a node of either is not
@@ -1184,6 +1184,30 @@ __global__ void copy_kernel(double* dst, const double* src, int64_t n) {
   if (i < n) dst[i] = src[i];
 }
 
+// one wave per instance, one lane per row of wave speeds
+__global__ __launch_bounds__(512) void publish_kernel(const PublishArgs a) {
+  const int lane = threadIdx.x % 64;
+  static_assert(kLamSlots == 64, "one lane per row");
+  if (a.lam) {
+    for (int i = threadIdx.x / 64; i < a.count; i += blockDim.x / 64) {
+      double* p = a.lam + (int64_t)lane * a.lam_ld + i;
+      double m = *p;
+      *p = 0.0;
+      for (int off = 32; off > 0; off >>= 1) {
+        const double o = __shfl_xor(m, off, 64);
+        m = o > m ? o : m;
+      }
+      if (lane == 0) a.lam_out[i] = m;
+    }
+  }
+  if (a.err && threadIdx.x < 4) a.err_out[threadIdx.x] = a.err[threadIdx.x];
+  if (a.n_active && threadIdx.x == 0) *a.n_active_out = *a.n_active;
+}
+
+hipError_t launch_publish(const PublishArgs& a, hipStream_t s) {
+  publish_kernel<<<1, a.lam && a.count > 1 ? 512 : 64, 0, s>>>(a);
+  return hipGetLastError();
+}
 hipError_t launch_fill(double* p, double v, int64_t n, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   fill_kernel<<<(n + 255) / 256, 256, 0, s>>>(p, v, n);

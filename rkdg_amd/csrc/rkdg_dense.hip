@@ -482,100 +482,153 @@ __global__ __launch_bounds__(256) void dense_means_kernel(const MeansArgs A, con
   for (int v = 0; v < NEQ; v++) A.means[v * A.NE + e] = s[v] / ms;
 }
 
-// Only the deciding variable's indicator is formed (density for the
+// Limiter. Only the deciding variable's indicator is formed (density for the
 // multiplier, indicator_bj.cpp:193; the last variable for FinDiff,
 // limiter_findiff.cpp:7-8).
+//
+// One lane per vertex: lane f of an element's T = 3 or 4 evaluates vertex f and
+// the two indicator points of edge f from the nodes staged in LDS, 21 triangles or
+// 16 quadrilaterals per wavefront. Teams sized for the right-hand side's points
+// (16 lanes for a P2 triangle) worked on 6 points and 3 vertices with 4 elements
+// per wavefront (120,540 P2 triangles: 23.5 -> 10.7 us; 473,000 Q1 quadrilaterals:
+// 44 -> 25 us; 27,467 Q2: 11.1 -> 6.6 us). An element whose factor is exactly 1 is
+// not written in place.
+template <int GEOM, int P>
+struct LDC : DC<GEOM, P> {
+  using D = DC<GEOM, P>;
+  static constexpr int T = D::NV;
+  static constexpr int EPB = 64 / T;
+  static constexpr int ROW = D::ND + (D::ND & 1);
+  // LDS stride of an element: the elements of a wavefront, which read the same
+  // node at once, start on different banks
+  static constexpr int ES = D::NEQ * ROW + (32 + 2 - (D::NEQ * ROW) % 32) % 32;
+  static constexpr int NTAB = (2 * D::NF + D::NV) * D::ND;  // PhiI, PhiV: the end of DenseTab
+};
+
+// minimum over the T lanes of an element (lane: its index)
+template <int T>
+__device__ __forceinline__ double vertex_min(double x, int lane) {
+  const int base = (int)(threadIdx.x % 64) - lane;
+  const double x0 = x;
+#pragma unroll
+  for (int k = 1; k < T; k++) {
+    const int src = lane + k < T ? lane + k : lane + k - T;
+    const double o = __shfl(x0, base + src, 64);
+    x = o < x ? o : x;
+  }
+  return x;
+}
+
 template <int GEOM, int P>
 __global__ __launch_bounds__(64, 4) void dense_limit_kernel(const LimitArgs A, const SchemeParams g,
                                                          const double* __restrict__ gtab) {
-  using C = DC<GEOM, P>;
-  constexpr int ND = C::ND, NEQ = C::NEQ, NF = C::NF, NV = C::NV;
-  constexpr int T = C::T, EPB = C::EPB, BLOCK = C::BLOCK;
-  constexpr int NPT = NF * 2;
+  using C = LDC<GEOM, P>;
+  constexpr int ND = C::ND, NEQ = C::NEQ, NF = C::NF, T = C::T, EPB = C::EPB;
+  constexpr int ROW = C::ROW, ES = C::ES, NTAB = C::NTAB;
 
-  __shared__ DenseTab<GEOM, P> tb;
-  __shared__ double s_u[EPB][NEQ][ND];
-  __shared__ double s_mean[EPB][NEQ];  // the element's means
-  __shared__ double s_nbm[EPB][NF];    // deciding variable's means of the face neighbours
-  __shared__ double s_area[EPB][ND];   // node mass weights (triangles: det J in [0])
+  __shared__ __attribute__((aligned(16))) double s_u[EPB * ES];  // [element][variable][node]
+  __shared__ double s_tab[NTAB];
+  __shared__ double s_mean[EPB][NEQ];
+  __shared__ double s_f[EPB];
+  __shared__ int s_on[EPB];
 
   const int tid = threadIdx.x;
-  const int team = tid / T, lane = tid % T;
+  const int team = tid / T, lane = tid - team * T;
   const int64_t NE = A.NE;
   const int64_t NDOFS = NE * ND;
   const int64_t e0 = xcd_remap_d(blockIdx.x, gridDim.x) * EPB;
   const int64_t e = e0 + team;
-  const bool active = e < NE && (!A.active || A.active[A.inst[e]]);
-  const int vsel = g.limiter == RKDG_LIM_FINDIFF ? NEQ - 1 : 0;
+  const bool in = team < EPB && e < NE;
+  const bool active = in && (!A.active || A.active[A.inst[e]]);
+  const bool multi = g.limiter == RKDG_LIM_MULTI, findiff = g.limiter == RKDG_LIM_FINDIFF;
+  const int vsel = findiff ? NEQ - 1 : 0;
 
   // every load of the setup is issued before the first LDS store
-  CopyRegs<sizeof(DenseTab<GEOM, P>) / sizeof(double), BLOCK> tbr;
-  tbr.load(gtab, tid);
-  StateRegs<EPB, NEQ, ND, BLOCK> str;
-  str.load(A.x, NDOFS, e0, NE, tid);
-  // the element's means (lane v < NEQ), the deciding variable's means of the
-  // face neighbours (lane f < NF) and the node mass weights (lane k < ND): one
-  // load instruction each, combined through LDS after the barrier
-  static_assert(NEQ <= T && NF <= T && ND <= T, "one lane per variable, face and node");
+  constexpr int LP = (EPB * ND + 63) / 64;
+  const int nn = (int)((NE - e0 < EPB ? NE - e0 : EPB) * ND);  // nodes of this block's elements
+  double st[LP][NEQ];
+#pragma unroll
+  for (int p = 0; p < LP; p++) {
+    const int i = tid + 64 * p;
+#pragma unroll
+    for (int v = 0; v < NEQ; v++) st[p][v] = i < nn ? sbase(A.x + (v * NDOFS + e0 * ND))[(unsigned)i] : 1.0;
+  }
+  CopyRegs<NTAB, 64> tbr;
+  tbr.load(gtab + (sizeof(DenseTab<GEOM, P>) / sizeof(double) - NTAB), tid);
+  // the element's means (lane v; three lanes hold four variables) and the
+  // deciding variable's mean across edge f = lane
+  static_assert(NF == T && NEQ <= T + 1, "one lane per vertex and edge");
   const bool ind_bj = g.indicator == RKDG_IND_BJ;
   const bool venkat = g.phi == RKDG_PHI_VENKAT && g.venkat_k > 0.0;
-  const double mown = (active && lane < NEQ) ? A.means[lane * NE + e] : 0.0;
-  const int nbl = (active && ind_bj && lane < NF) ? A.nbr[lane * NE + e] : -1;
+  const double mown = active ? A.means[lane * NE + e] : 0.0;
+  const double mlast = (NEQ > T && active && lane == 0) ? A.means[T * NE + e] : 0.0;
+  const int nbl = (active && ind_bj) ? A.nbr[lane * NE + e] : -1;
   const double nml = nbl >= 0 ? A.means[vsel * NE + nbl] : 0.0;
-  const unsigned long long nbb = __ballot(nbl >= 0);
-  const int nbmask = (int)((nbb >> (team * T)) & ((1ull << NF) - 1ull));  // bit f: face f has a neighbour
-  double arl = 0.0;
+  double eps2 = 0.0;
   if (active && venkat) {
-    if (C::TRI) arl = lane == 0 ? A.geo[(int64_t)C::G_DET * NE + e] : 0.0;
-    else arl = lane < ND ? A.geo[(int64_t)(C::G_MW + lane) * NE + e] : 0.0;
+    // (K h)^3 with h = |element|^(1/2); a quadrilateral's area from its edges,
+    // edge f running along (-n_1, n_0) of its area normal n
+    double area;
+    if (C::TRI) {
+      area = 0.5 * A.geo[(int64_t)C::G_DET * NE + e];
+    } else {
+      double n[6];
+#pragma unroll
+      for (int k = 0; k < 6; k++) n[k] = A.geo[(int64_t)(C::G_NRM + k) * NE + e];
+      const double d0 = n[0] + n[2], d1 = n[1] + n[3];  // the normal of the diagonal
+      area = 0.5 * ((n[0] * n[3] - n[1] * n[2]) + (d0 * n[5] - d1 * n[4]));
+    }
+    const double kh = g.venkat_k * sqrt(area);
+    eps2 = kh * kh * kh;
   }
-  tbr.store(reinterpret_cast<double*>(&tb), tid);
-  str.store(s_u, tid);
-  if (lane < NEQ) s_mean[team][lane] = mown;
-  if (lane < NF) s_nbm[team][lane] = nml;
-  if (lane < ND) s_area[team][lane] = arl;
+#pragma unroll
+  for (int p = 0; p < LP; p++) {
+    const int i = tid + 64 * p;
+    if (i < EPB * ND) {
+      const int el = i / ND, k = i - el * ND;
+#pragma unroll
+      for (int v = 0; v < NEQ; v++) s_u[el * ES + v * ROW + k] = st[p][v];
+    }
+  }
+  tbr.store(s_tab, tid);
+  if (team < EPB) {
+    s_mean[team][lane] = mown;
+    if (NEQ > T && lane == 0) s_mean[team][NEQ - 1] = mlast;
+  }
   __syncthreads();
   double mean[NEQ];
 #pragma unroll
-  for (int v = 0; v < NEQ; v++) mean[v] = s_mean[team][v];
+  for (int v = 0; v < NEQ; v++) mean[v] = s_mean[team < EPB ? team : 0][v];
+  const double msel = findiff ? mean[NEQ - 1] : mean[0];
   double mI = 1e9, MI = -1e9;
-  if (active && ind_bj) {
-    const double mv = mean[vsel];
-    mI = mv;
-    MI = mv;
-#pragma unroll
-    for (int f = 0; f < NF; f++) {
-      if ((nbmask >> f) & 1) {
-        const double a = s_nbm[team][f];
-        mI = a < mI ? a : mI;
-        MI = a > MI ? a : MI;
-      }
-    }
-  }
-  double eps2 = 0.0;
-  if (active && venkat) {
-    // (K h)^3 with h = |element|^(1/2)
-    double area = 0.0;
-    if (C::TRI) area = 0.5 * s_area[team][0];
-    else
-#pragma unroll
-      for (int k = 0; k < ND; k++) area += s_area[team][k];
-    const double h = sqrt(area);
-    const double kh = g.venkat_k * h;
-    eps2 = kh * kh * kh;
-  }
-  double ylane = 1e9;  // this lane's minimum over its indicator points
   if (ind_bj) {
-    for (int it = lane; it < NPT; it += T) {
-      if (!active) break;
-      const int f = it / 2, ip = it % 2;
-      double yc = 1e9;
-      if ((nbmask >> f) & 1) {
-        double u = 0.0;
+    // stencil bounds of the means: the cell and its edge neighbours
+    const double a = nbl >= 0 ? nml : msel;
+    mI = vertex_min<T>(a < msel ? a : msel, lane);
+    MI = -vertex_min<T>(-(a > msel ? a : msel), lane);
+  }
+  const double* ue = &s_u[(team < EPB ? team : 0) * ES];
+  const double* pv = &s_tab[2 * NF * ND + lane * ND];
+  double vs[NEQ];  // the state at the vertex
+  double yr = 1e9;
+  if (ind_bj) {
+    const double* p0 = &s_tab[2 * lane * ND];
+    const double* u = ue + vsel * ROW;
+    double pt[2] = {0.0, 0.0}, V = 0.0;
 #pragma unroll
-        for (int k = 0; k < ND; k++) u += s_u[team][vsel][k] * tb.PhiI[f][ip][k];
-        const double diff = u - mean[vsel];
-        const double y = indicator_y(diff, mean[vsel], mI, MI);
+    for (int k = 0; k < ND; k++) {
+      const double x = u[k];
+      pt[0] += x * p0[k];
+      pt[1] += x * p0[ND + k];
+      V += x * pv[k];
+    }
+    vs[0] = V;
+    if (nbl >= 0) {
+#pragma unroll
+      for (int ip = 0; ip < 2; ip++) {
+        const double diff = pt[ip] - msel;
+        const double y = indicator_y(diff, msel, mI, MI);
+        double yc;
         if (g.phi == RKDG_PHI_BJ) {
           yc = y < 1.0 ? y : 1.0;
         } else if (g.phi == RKDG_PHI_VENKAT) {
@@ -590,100 +643,88 @@ __global__ __launch_bounds__(64, 4) void dense_limit_kernel(const LimitArgs A, c
           const double yRel = y / yStar;
           yc = y < 1.0 ? y + (3.0 - 2.0 * yStar) * yRel * yRel + (yStar - 2.0) * yRel * yRel * yRel : 1.0;
         }
+        yr = yc < yr ? yc : yr;
       }
-      ylane = yc < ylane ? yc : ylane;
     }
+    yr = vertex_min<T>(yr, lane);
   }
-  // minimum over the team's lanes (min is exact, so the order does not matter)
-#pragma unroll
-  for (int off = T / 2; off > 0; off >>= 1) {
-    const double o = __shfl_xor(ylane, off, 64);
-    ylane = o < ylane ? o : ylane;
-  }
-  double yr = ylane;
   if (g.indicator == RKDG_IND_NOWHERE) yr = 1.0;
   else if (g.indicator == RKDG_IND_EVERYWHERE) yr = 0.0;
+
+  const bool linear = P == 1 && !C::TRI && g.linearize && multi;
   if constexpr (P == 1 && !C::TRI) {
     // linearize: the multiplier and the last hope work on the element's linear
-    // reconstruction (triangles are skipped, limiter_multiplier.cpp:29)
-    if (g.linearize && g.limiter == RKDG_LIM_MULTI) {
+    // reconstruction (triangles are skipped, limiter_multiplier.cpp:29); lane = node
+    if (linear) {
       double lin[NEQ];
-      const bool nl = active && lane < ND;
-      if (nl) {
 #pragma unroll
-        for (int v = 0; v < NEQ; v++) lin[v] = linearize_q1<2>(&s_u[team][v][0], mean[v], lane);
-      }
+      for (int v = 0; v < NEQ; v++) lin[v] = linearize_q1<2>(ue + v * ROW, mean[v], lane);
       __syncthreads();
-      if (nl) {
 #pragma unroll
-        for (int v = 0; v < NEQ; v++) s_u[team][v][lane] = lin[v];
-      }
+      for (int v = 0; v < NEQ; v++) s_u[team * ES + v * ROW + lane] = lin[v];
       __syncthreads();
     }
   }
-  const int j = lane;
-  const bool node_lane = active && lane < ND;
-  double u[NEQ];
-  if (node_lane) {
-#pragma unroll
-    for (int v = 0; v < NEQ; v++) u[v] = s_u[team][v][j];
-  }
   int trouble = 0;
-  if (g.limiter == RKDG_LIM_MULTI) {
+  double f = 1.0;  // the factor of the limited state mean + f (u - mean)
+  if (multi) {
     if (yr < 1.0) trouble = 1;
-    double f = yr;
+    f = yr;
     if (g.pow_nd) {
       double acc = 1.0, b = yr;
+#pragma unroll
       for (int e2 = ND; e2 > 0; e2 >>= 1) {
         if (e2 & 1) acc *= b;
         b *= b;
       }
       f = acc;
     }
-    if (node_lane) {
-#pragma unroll
-      for (int v = 0; v < NEQ; v++) u[v] = mean[v] + f * (u[v] - mean[v]);
-    }
     if (g.last_hope) {
-      bool bad_v = false;
-      for (int it = lane; it < NV; it += T) {
-        if (!active) break;
-        double vs[NEQ];
 #pragma unroll
-        for (int v = 0; v < NEQ; v++) {
-          double s = 0.0;
+      for (int v = 0; v < NEQ; v++) {
+        if (v > 0 || !ind_bj || linear) {
+          double V = 0.0;
 #pragma unroll
-          for (int k = 0; k < ND; k++) s += s_u[team][v][k] * tb.PhiV[it][k];
-          vs[v] = mean[v] + f * (s - mean[v]);
+          for (int k = 0; k < ND; k++) V += ue[v * ROW + k] * pv[k];
+          vs[v] = V;
         }
-        if (!physical<2>(vs, g)) bad_v = true;
+        vs[v] = mean[v] + f * (vs[v] - mean[v]);
       }
       // any unphysical vertex of the team's element (one ballot, no barrier)
-      const unsigned long long bm = __ballot(bad_v);
-      const unsigned long long tm = T == 64 ? ~0ull : (((1ull << T) - 1ull) << (team * T));
-      if (active && (bm & tm)) {
+      const unsigned long long bm = __ballot(active && !physical<2>(vs, g));
+      if (active && ((bm >> (team * T)) & ((1ull << T) - 1ull))) {
         trouble |= 2;
-        if (node_lane) {
+        f = 0.0;
+      }
+    }
+  } else if (findiff) {
+    if (yr < 0.999) {
+      trouble = 1;
+      f = 0.0;
+    }
+  }
+  if (A.troubled && active && lane == 0) A.troubled[e] = (int8_t)trouble;
+  if (team < EPB && lane == 0) {
+    s_f[team] = f;
+    s_on[team] = active && (A.out || f != 1.0 || linear);
+  }
+  __syncthreads();
+  double* dst = A.out ? A.out : A.x;
 #pragma unroll
-          for (int v = 0; v < NEQ; v++) u[v] = mean[v];
+  for (int p = 0; p < LP; p++) {
+    const int i = tid + 64 * p;
+    if (i < nn) {
+      const int el = i / ND, k = i - el * ND;
+      if (s_on[el]) {
+        const double fe = s_f[el];
+#pragma unroll
+        for (int v = 0; v < NEQ; v++) {
+          const double m = s_mean[el][v], u = s_u[el * ES + v * ROW + k];
+          sbase(dst + (v * NDOFS + e0 * ND))[(unsigned)i] = fe == 1.0 ? u : m + fe * (u - m);
         }
       }
     }
-  } else if (g.limiter == RKDG_LIM_FINDIFF) {
-    if (yr < 0.999) {
-      trouble = 1;
-      if (node_lane) {
-#pragma unroll
-        for (int v = 0; v < NEQ; v++) u[v] = mean[v];
-      }
-    }
   }
-  if (node_lane && (g.limiter != RKDG_LIM_NONE || A.out)) {
-    double* dst = A.out ? A.out : A.x;
-#pragma unroll
-    for (int v = 0; v < NEQ; v++) dst[v * NDOFS + e * ND + j] = u[v];
-  }
-  if (A.troubled && active && lane == 0) A.troubled[e] = (int8_t)trouble;
 }
 
 // ---------------------------------------------------------------------------
@@ -753,9 +794,9 @@ hipError_t launch_dense_limit(int geom, int p, const LimitArgs& a, const SchemeP
                               hipStream_t s) {
 #define X(G, PP)                                                                \
   if (geom == G && p == PP) {                                                   \
-    using C = DC<G, PP>;                                                        \
+    using C = LDC<G, PP>;                                                       \
     const int64_t nb = (a.NE + C::EPB - 1) / C::EPB;                            \
-    dense_limit_kernel<G, PP><<<(unsigned)nb, C::BLOCK, 0, s>>>(a, g, t);       \
+    dense_limit_kernel<G, PP><<<(unsigned)nb, 64, 0, s>>>(a, g, t);             \
     return hipGetLastError();                                                   \
   }
   RKDG_DENSE_CASES(X)

@@ -65,3 +65,39 @@ def test_limiter_block_edges(dim, order, kind, cuda):
             flags = fd.cpu().numpy()
             assert np.all(((flags & 1) == (ymin < 1.0)) | (np.abs(ymin - 1.0) < 1e-12)), (n, kind)
         ctx.close()
+
+
+@pytest.mark.parametrize("kind", list(KINDS))
+@pytest.mark.parametrize("geom,order", [("tri", 1), ("tri", 2), ("tri", 3), ("quad", 1), ("quad", 2), ("quad", 3)])
+def test_dense_limiter_block_edges(geom, order, kind, cuda):
+    """The dense limiter holds 21 triangles or 16 quadrilaterals per wavefront."""
+    import torch
+
+    from rkdg_amd.capi import Context
+
+    def bulge(X, Y):
+        return X + 0.04 * np.sin(3 * X) * np.cos(2 * Y), Y + 0.05 * np.sin(2 * X + Y)
+
+    sizes = ((2, 1), (5, 2), (7, 3), (3, 7), (9, 8)) if geom == "tri" else ((2, 1), (5, 3), (4, 4), (17, 1), (13, 9))
+    for nx, ny in sizes:
+        m = (M.jittered_delaunay_tri(nx, ny, 0.0, 1.0, 0.0, 1.0, seed=3) if geom == "tri"
+             else M.structured_quad(nx, ny, warp=bulge))
+        sch = S.Scheme(riemann=S.HLLC, indicator=S.IND_BJ, bcs=all_outlet(m), **KINDS[kind])
+        ref = RefSolver(m, order, sch)
+        xyz = ref.node_coords()
+        U = smooth_state(xyz, seed=9, amp=1e-4).reshape(4, -1)
+        j = (xyz[..., 0].ravel() > 0.55).astype(float)
+        U[0] *= 1.0 + 1.5 * j
+        U[-1] *= 1.0 + 2.5 * j
+        x = np.ascontiguousarray(U.reshape(-1))
+        x_ref, _, ymin = ref.limit(x)
+        ctx = Context(m, order, sch, dense=geom == "quad")
+        xd = torch.from_numpy(x).to(cuda)
+        fd = torch.full((m.num_elements,), 7, dtype=torch.int8, device=cuda)
+        ctx.limit(xd, fd)
+        err = np.abs(xd.cpu().numpy() - x_ref).reshape(4, -1).max(axis=1)
+        assert np.all(err <= 1e-12 * np.abs(U).max(axis=1)), (m.num_elements, kind)
+        if KINDS[kind]["limiter"] == S.LIM_MULTI:
+            flags = fd.cpu().numpy()
+            assert np.all(((flags & 1) == (ymin < 1.0)) | (np.abs(ymin - 1.0) < 1e-12)), (m.num_elements, kind)
+        ctx.close()

@@ -340,9 +340,10 @@ int rkdg_forward_solve(rkdg_ctx* ctx, double* x, int64_t nsteps, const double* d
                        const double* b, const double* c, int obj_slot, double* J);
 /* Gradient of that J with respect to the initial state x0 (x0bar) and the
  * boundary parameters (bc_param_bar, HOST [RKDG_MAX_BC*8]) for the fixed dt
- * schedule, by sqrt(N) checkpointing: checkpoints every `every` steps (0:
- * ceil(sqrt(nsteps))), each segment recomputed once with its stage states
- * recorded. J: HOST; xN (nullable): final state. */
+ * schedule, by checkpointing: checkpoints every `every` steps (0: none where
+ * the records of all steps fit 2 GiB, else ceil(sqrt(nsteps))), each segment
+ * but the last, which is recorded as it is taken, recomputed once with its
+ * stage states recorded. J: HOST; xN (nullable): final state. */
 int rkdg_adjoint_solve(rkdg_ctx* ctx, const double* x0, int64_t nsteps, const double* dts, int s,
                        const double* a, const double* b, const double* c, int obj_slot, int64_t every,
                        double* J, double* x0bar, double* bc_param_bar, double* xN);

@@ -38,7 +38,7 @@ RKDG_HD void zero(SideBar& b) {
 // converts the p, c, inv adjoints into state adjoints.
 RKDG_HD void finish_side(const double* s, const SchemeParams& g, SideBar& b) {
   const double rho = s[0];
-  const double inv = 1.0 / rho;
+  const double inv = recip(rho);
   const double m2 = s[1] * s[1] + s[2] * s[2];
   const double cg = g.gamma - 1.0;
   const double pid = cg * (s[3] - 0.5 * m2 * inv);
@@ -46,8 +46,7 @@ RKDG_HD void finish_side(const double* s, const SchemeParams& g, SideBar& b) {
   const double p = pid * f;
   if (b.c != 0.0) {
     const double a = g.gamma * p * inv * f;
-    const double c = sqrt(a);
-    const double abar = b.c / (2.0 * c);
+    const double abar = 0.5 * b.c * recip(sqrt_ws(a));
     b.p += abar * g.gamma * inv * f;
     b.inv += abar * g.gamma * p * f;
     if (g.covolume != 0.0) b.s[0] += abar * g.gamma * p * inv * g.covolume * f * f;
@@ -66,8 +65,9 @@ RKDG_HD void finish_side(const double* s, const SchemeParams& g, SideBar& b) {
 
 // u = s[1]/s[0] (a velocity formed by division)
 RKDG_HD void velocity_vjp(const double* s, double ubar, SideBar& b) {
-  b.s[1] += ubar / s[0];
-  b.s[0] += -ubar * s[1] / (s[0] * s[0]);
+  const double inv = recip(s[0]);
+  b.s[1] += ubar * inv;
+  b.s[0] += -ubar * s[1] * (inv * inv);
 }
 
 // contravariant volume flux G = a . F(u) at a node (the nodal flux of the
@@ -76,7 +76,7 @@ RKDG_HD void volume_flux_vjp(const double* s, const double* a, const double* Gba
                              double* sbar) {
   SideBar b;
   zero(b);
-  const double inv = 1.0 / s[0];
+  const double inv = recip(s[0]);
   const double m2 = s[1] * s[1] + s[2] * s[2];
   const double cg = g.gamma - 1.0;
   const double f = g.covolume != 0.0 ? 1.0 / (1.0 - s[0] * g.covolume) : 1.0;
@@ -105,7 +105,7 @@ RKDG_HD void volume_flux_vjp(const double* s, const double* a, const double* Gba
 
 // x-flux of a rotated state f = (m, u m + p, u m_y, u (E + p)), u = m * (1/rho)
 RKDG_HD void xflux_vjp(const double* s, double p, const double* fbar, SideBar& b) {
-  const double inv = 1.0 / s[0];
+  const double inv = recip(s[0]);
   const double u = s[1] * inv;
   b.s[1] += fbar[0];
   const double ubar = fbar[1] * s[1] + fbar[2] * s[2] + fbar[3] * (s[3] + p);
@@ -118,23 +118,23 @@ RKDG_HD void xflux_vjp(const double* s, double p, const double* fbar, SideBar& b
 }
 
 RKDG_HD double side_pressure(const double* s, const SchemeParams& g) {
-  const double inv = 1.0 / s[0];
+  const double inv = recip(s[0]);
   const double m2 = s[1] * s[1] + s[2] * s[2];
   double p = (g.gamma - 1.0) * (s[3] - 0.5 * m2 * inv);
   if (g.covolume != 0.0) p /= (1.0 - s[0] * g.covolume);
   return p;
 }
 RKDG_HD double side_sound_speed(const double* s, double p, const SchemeParams& g) {
-  double a = g.gamma * p / s[0];
+  double a = g.gamma * p * recip(s[0]);
   if (g.covolume != 0.0) a /= (1.0 - s[0] * g.covolume);
-  return sqrt(a);
+  return sqrt_ws(a);
 }
 
 // Toro two-rarefaction (or Einfeldt) speeds of rotated states: adjoint of (SL, SR)
 RKDG_HD void wave_speeds_vjp(const double* s1, const double* s2, double p1, double p2, const SchemeParams& g,
                              double SLbar, double SRbar, SideBar& b1, SideBar& b2) {
   const double cL = side_sound_speed(s1, p1, g), cR = side_sound_speed(s2, p2, g);
-  const double uL = s1[1] / s1[0], uR = s2[1] / s2[0];
+  const double uL = s1[1] * recip(s1[0]), uR = s2[1] * recip(s2[0]);
   double uLbar = 0.0, uRbar = 0.0;
   if (g.wave_speeds == RKDG_WS_EINFELDT) {
     const double sL = sqrt(s1[0]), sR = sqrt(s2[0]);
@@ -171,44 +171,40 @@ RKDG_HD void wave_speeds_vjp(const double* s1, const double* s2, double p1, doub
     b1.s[0] += sLbar / (2.0 * sL);
     b2.s[0] += sRbar / (2.0 * sR);
   } else {
-    const double gm = g.gamma;
-    const double z = 0.5 * (gm - 1.0) / gm;
-    const double pLz = pow(p1, z), pRz = pow(p2, z);
-    const double num = cL + cR - 0.5 * (gm - 1.0) * (uR - uL);
-    const double den = cL / pLz + cR / pRz;
-    const double r = num / den;
-    const double pStar = pow(r, 1.0 / z);
-    const double kap = 0.5 * (gm + 1.0) / gm;
-    const double qL = pStar > p1 ? sqrt(1.0 + kap * (pStar / p1 - 1.0)) : 1.0;
-    const double qR = pStar > p2 ? sqrt(1.0 + kap * (pStar / p2 - 1.0)) : 1.0;
+    // the same form as wave_speeds: r = pL/pR, P/pL = t = x^(1/z) with
+    // x = A / (cL + cR r^z), P/pR = t r, so the branches are those the forward took
+    const double hg = 0.5 * (g.gamma - 1.0), k = 1.0 - g.toro_z, z = g.toro_z;
+    const double ip2 = recip(p2);
+    const double r = p1 * ip2;
+    const double rz = pow_ws(r, z);
+    const double iD = recip(cL + cR * rz);
+    const double x = fmax((cL + cR - hg * (uR - uL)) * iD, g.toro_min);
+    const double t = g.toro_n ? pow_n(x, g.toro_n) : pow_ws(x, g.toro_iz);
+    const double tR = t * r;
     uLbar += SLbar;
-    const double qLbar = -SLbar * cL;
-    b1.c += -SLbar * qL;
     uRbar += SRbar;
-    const double qRbar = SRbar * cR;
+    const double qL = t > 1.0 ? sqrt_ws(1.0 + k * (t - 1.0)) : 1.0;
+    const double qR = tR > 1.0 ? sqrt_ws(1.0 + k * (tR - 1.0)) : 1.0;
+    b1.c += -SLbar * qL;
     b2.c += SRbar * qR;
-    double pStarbar = 0.0;
-    if (pStar > p1) {
-      const double t = qLbar * kap / (2.0 * qL);
-      pStarbar += t / p1;
-      b1.p += -t * pStar / (p1 * p1);
+    double tbar = 0.0, rbar = 0.0;
+    if (t > 1.0) tbar = -SLbar * cL * k * 0.5 * recip(qL);
+    if (tR > 1.0) {
+      const double tRbar = SRbar * cR * k * 0.5 * recip(qR);
+      tbar += tRbar * r;
+      rbar = tRbar * t;
     }
-    if (pStar > p2) {
-      const double t = qRbar * kap / (2.0 * qR);
-      pStarbar += t / p2;
-      b2.p += -t * pStar / (p2 * p2);
+    if (tbar != 0.0) {
+      const double xbar = tbar * t * recip(z * x);
+      const double Abar = xbar * iD, Dbar = -xbar * x * iD;
+      b1.c += Abar + Dbar;
+      b2.c += Abar + Dbar * rz;
+      uRbar += -hg * Abar;
+      uLbar += hg * Abar;
+      rbar += Dbar * cR * z * rz * recip(r);
     }
-    const double rbar = pStarbar * pStar / (z * r);
-    const double numbar = rbar / den;
-    const double denbar = -rbar * num / (den * den);
-    b1.c += numbar;
-    b2.c += numbar;
-    uRbar += -0.5 * (gm - 1.0) * numbar;
-    uLbar += 0.5 * (gm - 1.0) * numbar;
-    b1.c += denbar / pLz;
-    b2.c += denbar / pRz;
-    b1.p += denbar * cL * (-z) / (pLz * p1);
-    b2.p += denbar * cR * (-z) / (pRz * p2);
+    b1.p += rbar * ip2;
+    b2.p += -rbar * r * ip2;
   }
   velocity_vjp(s1, uLbar, b1);
   velocity_vjp(s2, uRbar, b2);
@@ -306,9 +302,10 @@ RKDG_HD void riemann_vjp(const SchemeParams& g, const double* uL, const double* 
     rot2(s2, n);
     rot2(Fr, n);  // adjoint of the inverse rotation of the flux
     const double p1 = side_pressure(s1, g), p2 = side_pressure(s2, g);
+    const double i1 = recip(s1[0]), i2 = recip(s2[0]);
     double f1[NE2], f2[NE2];
     {
-      const double u1 = s1[1] / s1[0], u2 = s2[1] / s2[0];
+      const double u1 = s1[1] * i1, u2 = s2[1] * i2;
       f1[0] = s1[1];
       f2[0] = s2[1];
       f1[1] = u1 * s1[1] + p1;
@@ -340,7 +337,7 @@ RKDG_HD void riemann_vjp(const SchemeParams& g, const double* uL, const double* 
       } else if (SR <= 0) {
         for (int i = 0; i < NE2; i++) f2bar[i] = Fr[i];
       } else {
-        const double inv = 1.0 / (SR - SL);
+        const double inv = recip(SR - SL);
         double invbar = 0.0;
         for (int i = 0; i < NE2; i++) {
           const double d = s2[i] - s1[i];
@@ -363,11 +360,12 @@ RKDG_HD void riemann_vjp(const SchemeParams& g, const double* uL, const double* 
       } else if (SR <= 0) {
         for (int i = 0; i < NE2; i++) f2bar[i] = Fr[i];
       } else {
-        const double gL = SL - s1[1] / s1[0];
-        const double gR = SR - s2[1] / s2[0];
+        const double gL = SL - s1[1] * i1;
+        const double gR = SR - s2[1] * i2;
         const double num = p2 - p1 + s1[1] * gL - s2[1] * gR;
         const double den = s1[0] * gL - s2[0] * gR;
-        const double sStar = num / den;
+        const double iden = recip(den);
+        const double sStar = num * iden;
         const bool left = sStar > 0.0;
         const double* st = left ? s1 : s2;
         const double* fK = left ? f1 : f2;
@@ -376,10 +374,11 @@ RKDG_HD void riemann_vjp(const SchemeParams& g, const double* uL, const double* 
         const double pK = left ? p1 : p2;
         const double SK = left ? SL : SR;
         const double gK = left ? gL : gR;
-        const double Wv = sStar - st[1] / st[0];
+        const double iK = left ? i1 : i2;
+        const double Wv = sStar - st[1] * iK;
         const double inner = pK + st[0] * gK * Wv;
         const double pterm = SK * inner;
-        const double inv = 1.0 / (SK - sStar);
+        const double inv = recip(SK - sStar);
         double invbar = 0.0, sStarbar = 0.0, SKbar = 0.0, ptermbar = 0.0;
         for (int i = 0; i < NE2; i++) {
           const double D = i == 1 ? 1.0 : (i == 3 ? sStar : 0.0);
@@ -402,10 +401,10 @@ RKDG_HD void riemann_vjp(const SchemeParams& g, const double* uL, const double* 
         double gKbar = innerbar * st[0] * Wv;
         const double Wvbar = innerbar * st[0] * gK;
         sStarbar += Wvbar;
-        bK.s[1] += -Wvbar / st[0];
-        bK.s[0] += Wvbar * st[1] / (st[0] * st[0]);
-        const double numbar = sStarbar / den;
-        const double denbar = -sStarbar * num / (den * den);
+        bK.s[1] += -Wvbar * iK;
+        bK.s[0] += Wvbar * st[1] * (iK * iK);
+        const double numbar = sStarbar * iden;
+        const double denbar = -numbar * sStar;
         b2.p += numbar;
         b1.p -= numbar;
         b1.s[1] += numbar * gL;
@@ -425,11 +424,11 @@ RKDG_HD void riemann_vjp(const SchemeParams& g, const double* uL, const double* 
         }
         gKbar = 0.0;
         SLbar += gLbar;
-        b1.s[1] -= gLbar / s1[0];
-        b1.s[0] += gLbar * s1[1] / (s1[0] * s1[0]);
+        b1.s[1] -= gLbar * i1;
+        b1.s[0] += gLbar * s1[1] * (i1 * i1);
         SRbar += gRbar;
-        b2.s[1] -= gRbar / s2[0];
-        b2.s[0] += gRbar * s2[1] / (s2[0] * s2[0]);
+        b2.s[1] -= gRbar * i2;
+        b2.s[0] += gRbar * s2[1] * (i2 * i2);
       }
     }
     if (SLbar != 0.0 || SRbar != 0.0) wave_speeds_vjp(s1, s2, p1, p2, g, SLbar, SRbar, b1, b2);

@@ -31,12 +31,13 @@ namespace rkdg {
 // element reads 2 NF doubles of its record, and the inverse mass is folded into
 // the volume and lift tables (triangles) or diagonal (quadrilaterals).
 //
-// Bound by FP64 issue and latency at 3 waves per SIMD. Limited steps, before
-// (power-of-two teams, every point reading the whole neighbour, dense inverse
-// mass and a full geometry record per element) and now: 27,467 bilinear Q2
-// quadrilaterals, two stages, HLLC 229 -> 108 us; 120,540 P2 triangles, three
-// stages, HLLC 488 -> 268 us; 472,000 Q1 quadrilaterals in 64 instances, eight
-// steps of three stages, HLL 12.9 -> 7.9 ms.
+// Bound by FP64 issue and latency at 3 to 5 waves per SIMD. Limited steps, at
+// first (power-of-two teams, every point reading the whole neighbour, dense
+// inverse mass and a full geometry record per element, the persistent loop) and
+// now, with the limiter's own change: 27,467 bilinear Q2 quadrilaterals, two
+// stages, HLLC 229 -> 70 us; 120,540 P2 triangles, three stages, HLLC 488 -> 187
+// us; 472,000 Q1 quadrilaterals in 64 instances, eight steps of three stages, HLL
+// 12.9 -> 4.4 ms.
 template <int GEOM, int P>
 struct RC : DC<GEOM, P> {
   using D = DC<GEOM, P>;
@@ -444,8 +445,14 @@ __device__ __forceinline__ void dense_rhs_block(const RhsArgs& A, const SchemePa
   __syncthreads();  // LDS is reused by the next work block
 }
 
-// persistent: the grid strides over the work blocks
-template <int GEOM, int P, int RS, bool BC>
+// One workgroup per work block, or (LOOP, when a grid cap below the number of
+// blocks is set) persistent: the grid strides over the work blocks. The loop keeps
+// the kernel's arguments in registers over its body, 143 to 165 VGPRs and 140 to
+// 175 spilled SGPRs against 90 to 99 (131 for P3 triangles) and 16 to 22 without
+// it, and a wave's tables are now too small for sharing them to pay: without it
+// the eight ensemble steps above take 4.4 instead of 5.5 ms, the Q2 step 70
+// instead of 83 us, the P2 step 187 instead of 207 us.
+template <int GEOM, int P, int RS, bool BC, bool LOOP>
 __global__ __launch_bounds__(64, 3) void dense_rhs_kernel(const RhsArgs A, const SchemeParams g,
                                                        const double* __restrict__ gtab, int64_t nvb) {
   __shared__ __attribute__((aligned(16))) DenseRhsTab<GEOM, P> tb;
@@ -453,6 +460,10 @@ __global__ __launch_bounds__(64, 3) void dense_rhs_kernel(const RhsArgs A, const
   tbr.load(gtab, threadIdx.x);
   tbr.store(reinterpret_cast<double*>(&tb), threadIdx.x);
   __syncthreads();
+  if constexpr (!LOOP) {
+    dense_rhs_block<GEOM, P, RS, BC>(A, g, xcd_remap_d(blockIdx.x, nvb), tb);
+    return;
+  }
   for (int64_t vb = blockIdx.x; vb < nvb; vb += gridDim.x) {
     // keep table reads inside the iteration (hoisted, they would hold registers across the loop)
     asm volatile("" ::: "memory");
@@ -765,9 +776,12 @@ hipError_t dense_rhs_rs(const RhsArgs& a, const SchemeParams& g, const double* t
   using C = RC<G, PP>;
   const int64_t nvb = (a.NE + C::EPB - 1) / C::EPB;
   const int64_t grid = a.grid_cap > 0 && a.grid_cap < nvb ? a.grid_cap : nvb;
-  if (bc) dense_rhs_kernel<G, PP, RS, true><<<(unsigned)grid, C::BLOCK, 0, s>>>(a, g, t, nvb);
-  else dense_rhs_kernel<G, PP, RS, false><<<(unsigned)grid, C::BLOCK, 0, s>>>(a, g, t, nvb);
-  return hipGetLastError();
+  auto launch = [&](auto kernel) {
+    kernel<<<(unsigned)grid, C::BLOCK, 0, s>>>(a, g, t, nvb);
+    return hipGetLastError();
+  };
+  if (grid < nvb) return launch(bc ? dense_rhs_kernel<G, PP, RS, true, true> : dense_rhs_kernel<G, PP, RS, false, true>);
+  return launch(bc ? dense_rhs_kernel<G, PP, RS, true, false> : dense_rhs_kernel<G, PP, RS, false, false>);
 }
 
 

@@ -246,8 +246,9 @@ RKDG_HD void rotate(double* s, const double* n) {
   } else {
     const double sp = n[2];
     const double cp = sqrt_ws(1 - sp * sp);
-    const double st = fabs(cp) > 1e-6 ? n[1] / cp : 1.0;
-    const double ct = fabs(cp) > 1e-6 ? n[0] / cp : 0.0;
+    const double ic = recip(cp);
+    const double st = fabs(cp) > 1e-6 ? n[1] * ic : 1.0;
+    const double ct = fabs(cp) > 1e-6 ? n[0] * ic : 0.0;
     double mx = cp * ct * m[0] + cp * st * m[1] + sp * m[2];
     double my = -st * m[0] + ct * m[1];
     double mz = -sp * ct * m[0] - sp * st * m[1] + cp * m[2];
@@ -269,8 +270,9 @@ RKDG_HD void inverse_rotate(double* s, const double* n) {
   } else {
     const double sp = n[2];
     const double cp = sqrt_ws(1 - sp * sp);
-    const double st = fabs(cp) > 1e-6 ? n[1] / cp : 1.0;
-    const double ct = fabs(cp) > 1e-6 ? n[0] / cp : 0.0;
+    const double ic = recip(cp);
+    const double st = fabs(cp) > 1e-6 ? n[1] * ic : 1.0;
+    const double ct = fabs(cp) > 1e-6 ? n[0] * ic : 0.0;
     double mx = cp * ct * m[0] - st * m[1] - sp * ct * m[2];
     double my = cp * st * m[0] + ct * m[1] - sp * st * m[2];
     double mz = sp * m[0] + cp * m[2];

@@ -15,9 +15,10 @@
 // processed one axis at a time (the -r and +r faces together): normal-direction
 // interpolation to face nodes, tangential interpolation to the face Gauss
 // points, Riemann solve, lift back. Every face flux is evaluated with the
-// arguments ordered as (Elem1 state, Elem2 state, Elem1 normal), so both
-// elements of a face see bitwise identical fluxes and the scheme is
-// conservative to round-off. Kernels are specialised on the Riemann solver and
+// arguments ordered as (Elem1 state, Elem2 state, Elem1 normal), or, for the
+// Rusanov flux on hexahedra, which has the symmetry bit by bit, with the own
+// side first and the outward normal: both elements of a face see bitwise
+// identical fluxes and the scheme is conservative to round-off. Kernels are specialised on the Riemann solver and
 // on the presence of boundary faces.
 #include <cstring>
 
@@ -189,6 +190,14 @@ __global__ __launch_bounds__(64, (ROLE == 1 ? 4 : rhs_waves<DIM, P, RS, BC, CV>(
   static_assert(!CV || (DIM == 3 && ROLE == 0 && !AL), "curved elements: 3D, one-kernel form, any orientation");
   using CL = CurvedLayout<P>;
   constexpr bool SOLVE = ROLE != 2;    // this kernel solves face fluxes
+  // Rusanov's flux is odd under the exchange of the sides with the normal's sign,
+  // in every rounding (each term is odd or even, the sums commute), so both
+  // elements may take it with their own side first and their outward normal and
+  // still see the same bits; the rotated solvers need the canonical order. It
+  // takes ten selects out of every face point (3032 Q2 hexahedra with hanging
+  // nodes: step 150 -> 142 us; the 96^3 step is bound by LDS and stays as it was).
+  // At order 3 it costs spills (Q3: 119 VGPRs and none -> 128 and 4 to 6)
+  constexpr bool OUTWARD = RS == RKDG_RS_RUSANOV && DIM == 3 && P <= 2;
   constexpr int ES = SOLVE ? EPB : 1;  // extent of the arrays only the face solves use
   constexpr int FB = NF * NEQ * NFN;   // lifted face fluxes of one receiver element
   __shared__ TT<C::N, C::NQ> tb;
@@ -291,10 +300,10 @@ __global__ __launch_bounds__(64, (ROLE == 1 ? 4 : rhs_waves<DIM, P, RS, BC, CV>(
 #pragma unroll
     for (int d = 0; d < DIM; d++) {
       const double nu = an[d] * inv;
-      s_nrm[team][f][d] = nu;
+      s_nrm[team][f][d] = OUTWARD && from_nb ? -nu : nu;
       nu2 += nu * nu;
     }
-    s_nrm[team][f][DIM] = sign * nmag;
+    s_nrm[team][f][DIM] = OUTWARD ? -nmag : sign * nmag;
     s_nrm[team][f][DIM + 1] = 0.5 * recip(sqrt_ws(nu2));
   }
   if (SOLVE && lane == 0 && team < ES) s_bad[team] = NF;
@@ -391,16 +400,14 @@ __global__ __launch_bounds__(64, (ROLE == 1 ? 4 : rhs_waves<DIM, P, RS, BC, CV>(
     // lift(r) + traces(r+1) | node accumulation(r) + points(r+1) ..., so each
     // axis costs two barriers.
     // Table values that depend on the lane but not on the axis: kept in registers
-    // over the axes (the phases below are one pass of the team when ONE_PASS)
-    // where they fit the registers of the waves asked for: at three waves, and in
-    // the aligned interior Rusanov form on Q2 hexahedra at four. The others read
-    // them from LDS again in each phase, 12 to 26 VGPRs less, which is what lets
-    // the rotated solvers on Q2 and Q3 hexahedra and the curved Rusanov form run
-    // at four (63,360 rotated Q2 hexahedra, HLL: step 642 -> 601 us; 29,760 curved
-    // ones, Rusanov: 481 -> 436 us; 29,667 Q3 hexahedra, LLF: 643 -> 624 us)
+    // over the axes (the phases below are one pass of the team when ONE_PASS) where
+    // the kernel runs at three waves and they fit. At four they are read from LDS
+    // again in each phase, 8 to 26 VGPRs less, which is what lets the rotated
+    // solvers on Q2 and Q3 hexahedra and the curved Rusanov form run at four (63,360
+    // rotated Q2 hexahedra, HLL: step 642 -> 601 us; 29,760 curved ones, Rusanov: 481
+    // -> 436 us; 29,667 Q3 hexahedra, LLF: 643 -> 624 us)
     constexpr bool ONE_PASS = 2 * NEQ * N <= T && 2 * NFP <= T;
-    constexpr bool TAB_REGS = ONE_PASS && ((ROLE == 0 && rhs_waves<DIM, P, RS, BC, CV>() == 3) ||
-                                           (AL && !BC && DIM == 3 && P == 2 && RS == RKDG_RS_RUSANOV));
+    constexpr bool TAB_REGS = ONE_PASS && ROLE == 0 && rhs_waves<DIM, P, RS, BC, CV>() == 3;
     double ec[N];         // traces: E[c][k] of the lane's face side
     double bqj[N];        // points: B[qj][b] of the lane's point
     double bqa[NQ];       // lift: B[qi][a] of the lane's row
@@ -509,7 +516,7 @@ __global__ __launch_bounds__(64, (ROLE == 1 ? 4 : rhs_waves<DIM, P, RS, BC, CV>(
           um[v] = t;
         }
         double nrm[DIM];
-        double snm, inm;  // -|n| on Elem1's side, +|n| on Elem2's; 0.5 / |unit normal|
+        double snm, inm;  // -|n| on Elem1's side (OUTWARD: on both), +|n| on Elem2's; 0.5 / |unit normal|
         if constexpr (CV) {
           // Elem1's normal at this point: the own record, or the neighbour's
           // at the point in its face frame
@@ -520,8 +527,8 @@ __global__ __launch_bounds__(64, (ROLE == 1 ? 4 : rhs_waves<DIM, P, RS, BC, CV>(
           const int qo = nb_first ? map_point<DIM, NQ>(code, qi, qj) : q;
           const double* fn = A.cgeo + eo * CL::size + CL::fn + (lfo * NFP + qo) * 5;
   #pragma unroll
-          for (int d = 0; d < DIM; d++) nrm[d] = fn[d];
-          snm = nb_first ? fn[DIM] : -fn[DIM];
+          for (int d = 0; d < DIM; d++) nrm[d] = OUTWARD && nb_first ? -fn[d] : fn[d];
+          snm = nb_first && !OUTWARD ? fn[DIM] : -fn[DIM];
           inm = fn[DIM + 1];
         } else {
   #pragma unroll
@@ -530,7 +537,6 @@ __global__ __launch_bounds__(64, (ROLE == 1 ? 4 : rhs_waves<DIM, P, RS, BC, CV>(
           inm = s_nrm[team][f][DIM + 1];
         }
         double fl[NEQ];
-        double factor = -1.0;
         bool ok = true;
         double lam = 0.0;
         if (!BC || nb >= 0) {
@@ -547,15 +553,18 @@ __global__ __launch_bounds__(64, (ROLE == 1 ? 4 : rhs_waves<DIM, P, RS, BC, CV>(
             }
             up[v] = t;
           }
-          factor = snm < 0.0 ? -1.0 : 1.0;
-          const bool elem1 = factor < 0.0;
-          double sL[NEQ], sR[NEQ];
+          if constexpr (OUTWARD) {
+            lam = riemann_t<DIM, RS>(g, um, up, nrm, fl, ok, inm);
+          } else {
+            const bool elem1 = snm < 0.0;
+            double sL[NEQ], sR[NEQ];
   #pragma unroll
-          for (int v = 0; v < NEQ; v++) {
-            sL[v] = elem1 ? um[v] : up[v];
-            sR[v] = elem1 ? up[v] : um[v];
+            for (int v = 0; v < NEQ; v++) {
+              sL[v] = elem1 ? um[v] : up[v];
+              sR[v] = elem1 ? up[v] : um[v];
+            }
+            lam = riemann_t<DIM, RS>(g, sL, sR, nrm, fl, ok, inm);
           }
-          lam = riemann_t<DIM, RS>(g, sL, sR, nrm, fl, ok, inm);
         } else if constexpr (BC) {
           const int slot = -1 - nb;
           if (slot < g.num_bc) {

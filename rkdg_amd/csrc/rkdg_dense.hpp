@@ -71,13 +71,6 @@ struct DenseRhsTab<GEOM, P, false> {
   double wq[NQ];
 };
 
-template <int GEOM, int P>
-__device__ __forceinline__ void stage_dense(DenseTab<GEOM, P>& d, const double* s) {
-  constexpr int n = sizeof(DenseTab<GEOM, P>) / sizeof(double);
-  double* o = reinterpret_cast<double*>(&d);
-  for (int i = threadIdx.x; i < n; i += blockDim.x) o[i] = s[i];
-}
-
 __device__ __forceinline__ int64_t xcd_remap_d(int64_t b, int64_t nb) {
   const int64_t q = nb / 8, r = nb % 8;
   const int64_t x = b % 8, l = b / 8;

@@ -37,7 +37,6 @@ struct TC {
   static constexpr int NFP = DIM == 3 ? NQ * NQ : NQ;
   static constexpr int NFN = DIM == 3 ? N * N : N;
   static constexpr int NVERT = DIM == 3 ? 8 : 4;
-  static constexpr int NIP = DIM == 3 ? 4 : 2;  // indicator points per face (order 2 rule)
   // lanes per element of the right-hand side. Q1 hexahedra: 20, which the 20
   // rows of the traces and the lift and the 18 points of an axis fill, so three
   // elements share a wavefront; 32 lanes held two of them and left 12 to 14 lanes

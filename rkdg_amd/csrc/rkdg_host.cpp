@@ -2003,7 +2003,12 @@ struct StepRec {
   double* mean[4];    // element means of v_1..v_s
 };
 
-constexpr int64_t kRecordBytes = int64_t(2) << 30;  // records of rkdg_adjoint_solve when it chooses
+// Records of rkdg_adjoint_solve when it chooses the segments: all steps up to 2 GiB,
+// and up to 48 GiB where that is at most a quarter of the free memory (2000 steps on
+// 16,128 Q1 quadrilaterals, 33 GB of records: gradient 334 ms, 399 in the call that
+// allocates them, against 423 with sqrt(N) segments)
+constexpr int64_t kRecordBytes = int64_t(2) << 30;
+constexpr int64_t kRecordBytesMax = int64_t(48) << 30;
 int rec_vectors(int s) { return 1 + s + (s - 1); }
 
 StepRec rec_at(rkdg_ctx* c, int s, size_t k) {
@@ -2836,14 +2841,32 @@ int rkdg_adjoint_solve(rkdg_ctx* c, const double* x0, int64_t N, const double* d
   if (!rc) rc = ensure_stage_buffers(c, 4);
   if (rc) return rc;
   // every = 0: record every step of the forward pass where the records fit
-  // kRecordBytes (then nothing is computed twice), else sqrt(N) checkpointing
+  // (then nothing is computed twice), else sqrt(N) checkpointing
   const int64_t step_bytes = (int64_t)(rec_vectors(s) + 1) * c->neq * c->ndofs * (int64_t)sizeof(double);
-  const int64_t K = every > 0                        ? std::min(every, N)
-                    : N * step_bytes <= kRecordBytes ? N
-                                                     : (int64_t)std::ceil(std::sqrt((double)N));
-  const int64_t ncp = (N + K - 1) / K;
+  const int64_t Kmin = (int64_t)std::ceil(std::sqrt((double)N));
+  int64_t K = every > 0 ? std::min(every, N) : Kmin;
+  if (every <= 0) {
+    const int64_t held = (int64_t)(c->d_rec.size() / (rec_vectors(s) + 1));
+    if (N <= std::max(held, kRecordBytes / step_bytes)) {
+      K = N;
+    } else if (N <= kRecordBytesMax / step_bytes) {
+      size_t avail = 0, total = 0;
+      HIP_TRY(hipMemGetInfo(&avail, &total));
+      if (N <= (int64_t)(avail / 4) / step_bytes) K = N;
+    }
+  }
+  const size_t slabs0 = c->d_rec_slabs.size(), recs0 = c->d_rec.size();
   rc = ensure_records(c, s, K);
+  if (rc == RKDG_E_HIP && every <= 0 && K > Kmin) {  // no memory for all: give back and take sqrt(N)
+    (void)hipGetLastError();
+    for (size_t i = slabs0; i < c->d_rec_slabs.size(); i++) dfree(c->d_rec_slabs[i]);
+    c->d_rec_slabs.resize(slabs0);
+    c->d_rec.resize(recs0);
+    K = Kmin;
+    rc = ensure_records(c, s, K);
+  }
   if (rc) return rc;
+  const int64_t ncp = (N + K - 1) / K;
   const int64_t sz = (int64_t)c->neq * c->ndofs;
   while ((int64_t)c->d_cp.size() < ncp + 1) {
     double* p = nullptr;

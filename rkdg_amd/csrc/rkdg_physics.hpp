@@ -373,42 +373,57 @@ template <int DIM, int RS>
 RKDG_HD double riemann_t(const SchemeParams& g, const double* uL, const double* uR, const double* n,
                          double* flux, bool& ok, double inm_face = 0.0) {
   constexpr int NE = DIM + 2;
+  if constexpr (RS == RKDG_RS_RUSANOV) {
+    // Every fused and every rounded product is written out and nothing else may be
+    // contracted: the two elements of a face may take the sides in either order, and
+    // a product fused into a sum of the sides (the build's default, left to itself,
+    // took the energy's) is exact on one side and rounded on the other.
+#pragma clang fp contract(off)
+    const double i1 = recip(uL[0]), i2 = recip(uR[0]);
+    double k1 = uL[1] * uL[1], k2 = uR[1] * uR[1], nm = n[0] * n[0];
+#pragma unroll
+    for (int d = 1; d < DIM; d++) {
+      k1 = fma(uL[1 + d], uL[1 + d], k1);
+      k2 = fma(uR[1 + d], uR[1 + d], k2);
+      nm = fma(n[d], n[d], nm);
+    }
+    const double pid1 = (g.gamma - 1.0) * fma(-0.5, k1 * i1, uL[1 + DIM]);
+    const double pid2 = (g.gamma - 1.0) * fma(-0.5, k2 * i2, uR[1 + DIM]);
+    ok = uL[0] >= 0.0 && uL[1 + DIM] > 0.0 && pid1 > 0.0 && uR[0] >= 0.0 && uR[1 + DIM] > 0.0 && pid2 > 0.0;
+    double p1 = pid1, p2 = pid2, c1 = g.gamma * pid1 * i1, c2 = g.gamma * pid2 * i2;  // pressures, c^2
+    if (g.covolume != 0.0) {
+      const double g1 = fma(-uL[0], g.covolume, 1.0), g2 = fma(-uR[0], g.covolume, 1.0);
+      p1 = pid1 / g1;
+      p2 = pid2 / g2;
+      c1 = g.gamma * p1 * i1 / g1;
+      c2 = g.gamma * p2 * i2 / g2;
+    }
+    const double m1 = fma(sqrt_ws(k1), i1, sqrt_ws(c1)), m2 = fma(sqrt_ws(k2), i2, sqrt_ws(c2));
+    const double mE = m1 > m2 ? m1 : m2;
+    // the unit normal's own norm (rs_rusanov.cpp:27-32); 1 up to rounding
+    const double inm = inm_face != 0.0 ? inm_face : 0.5 * recip(sqrt_ws(nm));
+    const double hm = 0.5 * mE;
+    double v1 = uL[1] * n[0], v2 = uR[1] * n[0];
+#pragma unroll
+    for (int d = 1; d < DIM; d++) {
+      v1 = fma(uL[1 + d], n[d], v1);
+      v2 = fma(uR[1 + d], n[d], v2);
+    }
+    const double a1 = v1 * i1, a2 = v2 * i2;
+    flux[0] = fma(-hm, uR[0] - uL[0], (v1 + v2) * inm);
+#pragma unroll
+    for (int d = 0; d < DIM; d++)
+      flux[1 + d] =
+          fma(-hm, uR[1 + d] - uL[1 + d], (fma(a1, uL[1 + d], p1 * n[d]) + fma(a2, uR[1 + d], p2 * n[d])) * inm);
+    flux[1 + DIM] = fma(-hm, uR[1 + DIM] - uL[1 + DIM], (a1 * (uL[1 + DIM] + p1) + a2 * (uR[1 + DIM] + p2)) * inm);
+    return mE;
+  } else {
   double s1[NE], s2[NE], f1[NE], f2[NE];
 #pragma unroll
   for (int i = 0; i < NE; i++) {
     s1[i] = uL[i];
     s2[i] = uR[i];
   }
-  if constexpr (RS == RKDG_RS_RUSANOV) {
-    const SidePrim<DIM> q1 = side_prim<DIM>(s1, g), q2 = side_prim<DIM>(s2, g);
-    ok = side_ok<DIM>(s1, q1) && side_ok<DIM>(s2, q2);
-    const double m1 = sqrt_ws(q1.m2) * q1.inv + side_sound<DIM>(s1, q1, g);
-    const double m2 = sqrt_ws(q2.m2) * q2.inv + side_sound<DIM>(s2, q2, g);
-    const double mE = m1 > m2 ? m1 : m2;
-    double vn1 = 0.0, vn2 = 0.0, nm = 0.0;
-#pragma unroll
-    for (int d = 0; d < DIM; d++) {
-      vn1 += s1[1 + d] * n[d];
-      vn2 += s2[1 + d] * n[d];
-      nm += n[d] * n[d];
-    }
-    const double a1 = vn1 * q1.inv, a2 = vn2 * q2.inv;
-    f1[0] = vn1;
-    f2[0] = vn2;
-#pragma unroll
-    for (int d = 0; d < DIM; d++) {
-      f1[1 + d] = a1 * s1[1 + d] + q1.p * n[d];
-      f2[1 + d] = a2 * s2[1 + d] + q2.p * n[d];
-    }
-    f1[1 + DIM] = a1 * (s1[1 + DIM] + q1.p);
-    f2[1 + DIM] = a2 * (s2[1 + DIM] + q2.p);
-    // the unit normal's own norm (rs_rusanov.cpp:27-32); 1 up to rounding
-    const double inm = inm_face != 0.0 ? inm_face : 0.5 * recip(sqrt_ws(nm));
-    const double hm = 0.5 * mE;
-#pragma unroll
-    for (int i = 0; i < NE; i++) flux[i] = (f1[i] + f2[i]) * inm - hm * (s2[i] - s1[i]);
-    return mE;
-  } else {
   rotate<DIM>(s1, n);
   rotate<DIM>(s2, n);
   const SidePrim<DIM> q1 = side_prim<DIM>(s1, g), q2 = side_prim<DIM>(s2, g);

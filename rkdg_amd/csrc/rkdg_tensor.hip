@@ -190,8 +190,9 @@ __global__ __launch_bounds__(64, (ROLE == 1 ? 4 : rhs_waves<DIM, P, RS, BC, CV>(
   using CL = CurvedLayout<P>;
   constexpr bool SOLVE = ROLE != 2;    // this kernel solves face fluxes
   // Rusanov's flux is odd under the exchange of the sides with the normal's sign,
-  // in every rounding (each term is odd or even, the sums commute), so both
-  // elements may take it with their own side first and their outward normal and
+  // in every rounding (each term is odd or even, the sums commute, and riemann_t
+  // fuses no product of one side into a sum of the two), so both elements
+  // may take it with their own side first and their outward normal and
   // still see the same bits; the rotated solvers need the canonical order. It
   // takes ten selects out of every face point (3032 Q2 hexahedra with hanging
   // nodes: step 150 -> 142 us; the 96^3 step is bound by LDS and stays as it was).

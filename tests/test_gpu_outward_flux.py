@@ -1,11 +1,11 @@
 """The Rusanov flux on hexahedra is taken outward from each element (its own side
 first) up to order 2 and in the face's order above: rotated elements, walls and
 periodic faces, against the oracle (relative L-infinity per variable <= 1e-12), and
-the two sides' shares against each other: with x = const + perturbation on a
-periodic mesh the integral of the right-hand side is the sum of face terms that
-cancel in pairs, so what is left is rounding of the sum, below 64 eps of the sum of
-the magnitudes (each of up to 27 * 64 terms is rounded a few times, and the errors
-of a sum of n terms grow like sqrt(n))."""
+conservation: on a periodic mesh the integral of the right-hand side is a sum of face
+terms that cancel in pairs, so what is left is rounding of the sum, below 64 eps of
+the sum of the magnitudes (each of up to 27 * 64 terms is rounded a few times, and
+the errors of a sum of n terms grow like sqrt(n)). That the two elements see the same
+bits is test_flux_pairs.py's."""
 import numpy as np
 import pytest
 

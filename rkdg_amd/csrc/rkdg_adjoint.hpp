@@ -179,7 +179,7 @@ RKDG_HD void wave_speeds_vjp(const double* s1, const double* s2, double p1, doub
     const double rz = pow_ws(r, z);
     const double iD = recip(cL + cR * rz);
     const double x = fmax((cL + cR - hg * (uR - uL)) * iD, g.toro_min);
-    const double t = g.toro_n ? pow_n(x, g.toro_n) : pow_ws(x, g.toro_iz);
+    const double t = toro_power(x, g);
     const double tR = t * r;
     uLbar += SLbar;
     uRbar += SRbar;

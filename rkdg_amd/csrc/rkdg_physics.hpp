@@ -325,6 +325,12 @@ RKDG_HD double pow_n(double x, int n) {
   return r;
 }
 
+// x^(1/z) of Toro's estimate: 0 for a base that has no power (a general power is
+// formed for positive bases only)
+RKDG_HD double toro_power(double x, const SchemeParams& g) {
+  return g.toro_n ? pow_n(x, g.toro_n) : (x > 0.0 ? pow_ws(x, g.toro_iz) : 0.0);
+}
+
 // Toro two-rarefaction speeds (physics.cpp:309-350) or Einfeldt (:269-296) on
 // rotated states; lo/hi = lambdaF[0], lambdaF[dim+1].
 //
@@ -355,9 +361,9 @@ RKDG_HD void wave_speeds(const double* s1, const double* s2, const SidePrim<DIM>
   const double r = q1.p * recip(q2.p);
   const double x =
       fmax((cL + cR - 0.5 * (gm - 1.0) * (uR - uL)) * recip(cL + cR * pow_ws(r, g.toro_z)), g.toro_min);
-  const double tL = g.toro_n ? pow_n(x, g.toro_n) : pow_ws(x, g.toro_iz);  // P / pL
-  const double tR = tL * r;                                               // P / pR
-  const double k = 1.0 - g.toro_z;                                        // (gamma+1)/(2 gamma)
+  const double tL = toro_power(x, g);  // P / pL
+  const double tR = tL * r;            // P / pR
+  const double k = 1.0 - g.toro_z;     // (gamma+1)/(2 gamma)
   const double qL = tL > 1.0 ? sqrt_ws(1.0 + k * (tL - 1.0)) : 1.0;
   const double qR = tR > 1.0 ? sqrt_ws(1.0 + k * (tR - 1.0)) : 1.0;
   lo = uL - qL * cL;

@@ -178,7 +178,8 @@ RKDG_HD void wave_speeds_vjp(const double* s1, const double* s2, double p1, doub
     const double r = p1 * ip2;
     const double rz = pow_ws(r, z);
     const double iD = recip(cL + cR * rz);
-    const double x = fmax((cL + cR - hg * (uR - uL)) * iD, g.toro_min);
+    double x = fmax((cL + cR - hg * (uR - uL)) * iD, g.toro_min);
+    if (toro_none(p1, p2, g)) x = 0.0;
     const double t = toro_power(x, g);
     const double tR = t * r;
     uLbar += SLbar;

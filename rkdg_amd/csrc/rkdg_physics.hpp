@@ -331,6 +331,14 @@ RKDG_HD double toro_power(double x, const SchemeParams& g) {
   return g.toro_n ? pow_n(x, g.toro_n) : (x > 0.0 ? pow_ws(x, g.toro_iz) : 0.0);
 }
 
+// A state denser than the covolume has a negative pressure and passes the state
+// check, which ignores the covolume (physics.cpp:84): the reference's powers of it are
+// no numbers and its comparisons take the acoustic speeds, as a base of 0 does here.
+// (Both pressures negative would have a ratio, and a sound speed, like any other.)
+RKDG_HD bool toro_none(double p1, double p2, const SchemeParams& g) {
+  return g.covolume != 0.0 && !(p1 > 0.0 && p2 > 0.0);
+}
+
 // Toro two-rarefaction speeds (physics.cpp:309-350) or Einfeldt (:269-296) on
 // rotated states; lo/hi = lambdaF[0], lambdaF[dim+1].
 //
@@ -359,8 +367,9 @@ RKDG_HD void wave_speeds(const double* s1, const double* s2, const SidePrim<DIM>
   const double cL = sqrt_ws(aL), cR = sqrt_ws(aR);
   const double gm = g.gamma;
   const double r = q1.p * recip(q2.p);
-  const double x =
+  double x =
       fmax((cL + cR - 0.5 * (gm - 1.0) * (uR - uL)) * recip(cL + cR * pow_ws(r, g.toro_z)), g.toro_min);
+  if (toro_none(q1.p, q2.p, g)) x = 0.0;
   const double tL = toro_power(x, g);  // P / pL
   const double tR = tL * r;            // P / pR
   const double k = 1.0 - g.toro_z;     // (gamma+1)/(2 gamma)

@@ -962,8 +962,11 @@ __global__ __launch_bounds__(64, 2) void tensor_limit_kernel(const LimitArgs A, 
   const bool ind_bj = g.indicator == RKDG_IND_BJ;
   const double mown = (active && lane < NEQ) ? A.means[lane * NE + e] : 0.0;
   const int nbl = (active && ind_bj && lane < NF) ? A.nbr[lane * NE + e] : -1;
-  double nml = nbl >= 0 ? A.means[vsel * NE + nbl] : 1e300;
-  double nmh = nbl >= 0 ? nml : -1e300;
+  // a neighbour whose mean is not a number bounds nothing (team_min would carry it
+  // to some of the lanes)
+  const double nm = nbl >= 0 ? A.means[vsel * NE + nbl] : NAN;
+  double nml = nm == nm ? nm : 1e300;
+  double nmh = nm == nm ? nm : -1e300;
   bool has_nb = nbl >= 0;
   if (A.ncnb && nbl <= kNcCode0) {  // a non-conforming face: the bounds over its neighbours
     const int k = kNcCode0 - nbl;

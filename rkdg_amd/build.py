@@ -60,9 +60,9 @@ def build(verbose: bool = False) -> str:
 def build_callers(verbose: bool = False) -> None:
     """The compiled programs that the tests run: a C program on the plain header
     (gcc) and a C++ program on the class mirror include/rkdg.hpp (hipcc for the HIP
-    runtime's allocation calls), which link librkdg.so, and two that evaluate the
-    device code's fluxes and wave speeds, flux_pairs with fused multiply-adds in its
-    host half as well."""
+    runtime's allocation calls), which link librkdg.so, as does a third that lets HIP
+    calls fail, and two that evaluate the device code's fluxes and wave speeds,
+    flux_pairs with fused multiply-adds in its host half as well."""
     root = os.path.dirname(HERE)
     capi = os.path.join(root, "tests", "capi")
     if not os.path.isdir(capi):
@@ -73,6 +73,8 @@ def build_callers(verbose: bool = False) -> None:
           "-o", os.path.join(capi, "capi_smoke")], verbose)
     _run([HIPCC, *FLAGS, "-Wall", *inc, os.path.join(capi, "cpp_smoke.cpp"), *link,
           "-o", os.path.join(capi, "cpp_smoke")], verbose)
+    _run([HIPCC, *FLAGS, "-Wall", *inc, os.path.join(capi, "hip_faults.cpp"), *link, "-ldl",
+          "-o", os.path.join(capi, "hip_faults")], verbose)
     _run([HIPCC, *FLAGS, "-Wall", "-Xarch_host", "-mfma", *inc, os.path.join(capi, "flux_pairs.hip"),
           "-o", os.path.join(capi, "flux_pairs")], verbose)
     _run([HIPCC, *FLAGS, "-Wall", *inc, os.path.join(capi, "toro_base.hip"),

@@ -1685,10 +1685,18 @@ hipError_t ensure_pinned(rkdg_ctx* c) {
 }
 double* pinned_lambda(rkdg_ctx* c) { return reinterpret_cast<double*>(c->h_pin + kPinWords); }
 
+// clears wave speeds that an earlier call left when it failed between its launch
+// and its reading
+int clear_lambda(rkdg_ctx* c) {
+  if (c->lam_dirty) HIP_TRY(launch_fill(c->d_lam, 0.0, (int64_t)kLamSlots * lam_stride(c->count), c->stream));
+  c->lam_dirty = false;
+  return RKDG_OK;
+}
+
 // the launch of `a` adds its wave speeds to d_lam
 int want_lambda(rkdg_ctx* c, RhsArgs& a) {
-  if (c->lam_dirty)  // an earlier call failed between its launch and its reading
-    HIP_TRY(launch_fill(c->d_lam, 0.0, (int64_t)kLamSlots * a.lam_ld, c->stream));
+  const int rc = clear_lambda(c);
+  if (rc) return rc;
   c->lam_dirty = true;
   a.no_lambda = 0;
   return RKDG_OK;
@@ -2530,10 +2538,10 @@ int rkdg_step_noalloc(rkdg_ctx* c, double* x, double t, double dt, int s, const 
     PublishArgs p{};
     p.lam = c->d_lam;
     p.lam_ld = lam_stride(c->count);
-    p.count = 1;
+    p.count = c->count;  // 1: a batch context has no scratch array
     p.lam_out = lambda_dev;
     HIP_TRY(launch_publish(p, c->stream));
-    c->lam_dirty = c->count > 1;  // a batch context: the other instances' words are still set
+    c->lam_dirty = false;
   }
   return RKDG_OK;
 }
@@ -3092,6 +3100,8 @@ int rkdg_batch_advance(rkdg_ctx* c, double* x, int s, const double* a, const dou
   Restore<bool> keep_prof(c->prof);
   HIP_TRY(hipStreamSynchronize(c->stream));
   c->stream = c->bstream;
+  rc = clear_lambda(c);  // here, not in the captured step: its replays clear nothing but what they read
+  if (rc) return rc;
   std::vector<double> key;
   key.push_back((double)(uintptr_t)x);
   key.push_back(s);

@@ -341,8 +341,8 @@ int rkdg_forward_solve(rkdg_ctx* ctx, double* x, int64_t nsteps, const double* d
 /* Gradient of that J with respect to the initial state x0 (x0bar) and the
  * boundary parameters (bc_param_bar, HOST [RKDG_MAX_BC*8]) for the fixed dt
  * schedule, by checkpointing: checkpoints every `every` steps (0: none where
- * the records of all steps fit 2 GiB, or 48 GiB and a quarter of the free
- * memory; the context holds them; else ceil(sqrt(nsteps))), each segment
+ * the records of all steps fit 2 GiB and a quarter of the free memory; the
+ * context holds them; else ceil(sqrt(nsteps))), each segment
  * but the last, which is recorded as it is taken, recomputed once with its
  * stage states recorded. J: HOST; xN (nullable): final state. */
 int rkdg_adjoint_solve(rkdg_ctx* ctx, const double* x0, int64_t nsteps, const double* dts, int s,

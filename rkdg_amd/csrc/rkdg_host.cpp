@@ -2011,12 +2011,12 @@ struct StepRec {
   double* mean[4];    // element means of v_1..v_s
 };
 
-// Records of rkdg_adjoint_solve when it chooses the segments: all steps up to 2 GiB,
-// and up to 48 GiB where that is at most a quarter of the free memory (2000 steps on
-// 16,128 Q1 quadrilaterals, 33 GB of records: gradient 334 ms, 399 in the call that
-// allocates them, against 423 with sqrt(N) segments)
+// Records of rkdg_adjoint_solve when it chooses the segments: all steps where they
+// fit 2 GiB and a quarter of the free memory. The context holds them, so more would
+// be missed by whatever else runs on the card: the 2000 steps of 16,128 Q1
+// quadrilaterals take 28.9 GB (gradient 332 ms, in the call that allocates them 387,
+// against 421 with sqrt(N) segments), and giving them back takes 80 ms or more.
 constexpr int64_t kRecordBytes = int64_t(2) << 30;
-constexpr int64_t kRecordBytesMax = int64_t(48) << 30;
 int rec_vectors(int s) { return 1 + s + (s - 1); }
 
 StepRec rec_at(rkdg_ctx* c, int s, size_t k) {
@@ -2832,9 +2832,9 @@ int rkdg_forward_solve(rkdg_ctx* c, double* x, int64_t nsteps, const double* dts
 // (last first) a recomputation recording the stage states and the reverse
 // sweep through it; the last segment is recorded in the forward pass itself:
 // 2N - K forward steps and N adjoint steps, K recorded steps and N/K checkpoints
-// resident. By default K = N where N records fit 2 GiB (16,128 Q1 quadrilaterals,
-// three stages: 148 steps; the gradient through 9 steps 2.06 -> 1.45 ms with
-// the derivatives below on reciprocals), else ceil(sqrt(N)).
+// resident. By default K = N where N records fit (kRecordBytes; 16,128 Q1
+// quadrilaterals, three stages: 148 steps; the gradient through 9 steps 2.06 ->
+// 1.45 ms with the derivatives below on reciprocals), else ceil(sqrt(N)).
 int rkdg_adjoint_solve(rkdg_ctx* c, const double* x0, int64_t N, const double* dts, int s, const double* a,
                        const double* b, const double* cc, int obj_slot, int64_t every, double* J, double* x0bar,
                        double* bc_param_bar, double* xN) {
@@ -2855,13 +2855,9 @@ int rkdg_adjoint_solve(rkdg_ctx* c, const double* x0, int64_t N, const double* d
   int64_t K = every > 0 ? std::min(every, N) : Kmin;
   if (every <= 0) {
     const int64_t held = (int64_t)(c->d_rec.size() / (rec_vectors(s) + 1));
-    if (N <= std::max(held, kRecordBytes / step_bytes)) {
-      K = N;
-    } else if (N <= kRecordBytesMax / step_bytes) {
-      size_t avail = 0, total = 0;
-      HIP_TRY(hipMemGetInfo(&avail, &total));
-      if (N <= (int64_t)(avail / 4) / step_bytes) K = N;
-    }
+    size_t avail = 0, total = 0;
+    if (N > held && N <= kRecordBytes / step_bytes) HIP_TRY(hipMemGetInfo(&avail, &total));
+    if (N <= held || N <= std::min(kRecordBytes, (int64_t)(avail / 4)) / step_bytes) K = N;
   }
   const size_t slabs0 = c->d_rec_slabs.size(), recs0 = c->d_rec.size();
   rc = ensure_records(c, s, K);

@@ -4,9 +4,10 @@
 //
 //   hip_faults batch       a read-back of the wave speeds fails between its two launches;
 //                          the ensemble's next steps must not see the abandoned speeds
-//   hip_faults records     memory runs out while an adjoint solve allocates its records;
-//                          it must take checkpoints instead, give the memory back and
-//                          return the same bits
+//   hip_faults records     memory runs out while an adjoint solve allocates its records,
+//                          or they are more than a quarter of what is free; it must take
+//                          checkpoints instead, give back what it took and return the
+//                          same bits
 #include <dlfcn.h>
 #include <hip/hip_runtime.h>
 
@@ -22,6 +23,7 @@ static hipError_t g_pending = hipSuccess;
 static size_t g_fail_size = 0;    // of the allocations of this size, counted from 0,
 static int g_fail_alloc = -1;     // the one that fails
 static int g_allocs = 0, g_failed = 0;
+static size_t g_free = 0;         // the free memory to report (0: what there is)
 
 template <typename F>
 static F real(const char* name) {
@@ -48,6 +50,12 @@ hipError_t hipMalloc(void** p, size_t n) {
     return hipErrorOutOfMemory;
   }
   return fn(p, n);
+}
+hipError_t hipMemGetInfo(size_t* avail, size_t* total) {
+  static auto fn = real<hipError_t (*)(size_t*, size_t*)>("hipMemGetInfo");
+  const hipError_t e = fn(avail, total);
+  if (g_free) *avail = g_free;
+  return e;
 }
 }
 
@@ -129,8 +137,9 @@ static int batch() {
   return 0;
 }
 
-// gradient through 30 steps; the allocation of record `fail` (-1: none) fails
-static int gradient(int fail, std::vector<double>& out) {
+// gradient through 30 steps; the allocation of record `fail` (-1: none) fails; the records of `room`
+// steps (0: any number) are a quarter of the free memory
+static int gradient(int fail, int room, std::vector<double>& out) {
   rkdg_ctx* c = nullptr;
   CHECK(rkdg_create_ex(&g_case.mesh, &g_case.scheme, RKDG_CREATE_DENSE, &c) == RKDG_OK);
   rkdg_info in;
@@ -143,14 +152,15 @@ static int gradient(int fail, std::vector<double>& out) {
   double J = 0.0, pbar[RKDG_MAX_BC * 8];
   g_fail_size = sizeof(double) * in.state_size * 7;  // one recorded step of three stages
   g_fail_alloc = fail;
+  g_free = 4 * g_fail_size * room;
   g_allocs = g_failed = 0;
   const int rc = rkdg_adjoint_solve(c, x, steps, dts.data(), 3, kA, kB, kC, 0, 0, &J, xbar, pbar, nullptr);
   const int allocs = g_allocs, failed = g_failed;
-  g_fail_size = 0;
+  g_fail_size = g_free = 0;
   CHECK(rc == RKDG_OK);
   CHECK(failed == (fail >= 0));
-  // every step's record, or, after the failure, those of one segment of six steps
-  CHECK(allocs == (fail >= 0 ? fail + 1 + 6 : steps));
+  // every step's record, or those of one segment of six steps, at once or after the failure
+  CHECK(allocs == (room > 0 && room < steps ? 6 : fail >= 0 ? fail + 1 + 6 : steps));
   out = host(xbar, (size_t)in.state_size);
   out.push_back(J);
   (void)hipFree(x);
@@ -161,9 +171,13 @@ static int gradient(int fail, std::vector<double>& out) {
 
 static int records() {
   std::vector<double> want, got;
-  if (gradient(-1, want)) return 1;
+  if (gradient(-1, 0, want)) return 1;
   for (int fail : {0, 1, 7, 29}) {
-    if (gradient(fail, got)) return 1;
+    if (gradient(fail, 0, got)) return 1;
+    CHECK(got == want);
+  }
+  for (int room : {1, 29, 30}) {
+    if (gradient(-1, room, got)) return 1;
     CHECK(got == want);
   }
   return 0;

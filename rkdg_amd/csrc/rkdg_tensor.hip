@@ -805,39 +805,44 @@ __global__ __launch_bounds__(64, (ROLE == 1 ? 4 : rhs_waves<DIM, P, RS, BC, CV>(
 
 // ---------------------------------------------------------------------------
 // element means (Averager::computeMeanValues): sum_k w_k u_k / sum_k w_k (det J
-// is constant on an affine element and cancels). A workgroup stages the states
-// of EB elements through LDS with coalesced loads, then one lane per (element,
-// variable) forms the sum: bound by the read of the state. The tree of shuffles
-// over an element's lanes that this replaces issued ten per variable and ran at
-// half the copy rate (96^3 Q2 hexahedra: 300 -> 225 us; 63 x 65 x 61 just
-// after the limiter wrote them, from the caches: 97 -> 64 us).
+// is constant on an affine element and cancels). A workgroup of NEQ wavefronts
+// stages the states of EB elements through LDS with coalesced loads; wavefront v
+// then sums variable v, S lanes per element with A partial sums each: bound by the
+// read of the state on large meshes, by latency on small ones. The short sums keep
+// the rounding error of a tree (1.7e-16 of the mean on 27 nodes, 8.5e-17 on 64; one
+// serial sum per lane 2.5e-16 and 6.2e-16) and a short chain. A tree of shuffles with
+// one lane per node, the serial sum, now: 96^3 Q2 hexahedra 311, 207, 198 us; 40^3 Q3
+// 53, 33, 25 us; 729 Q3 3.2, 3.9, 3.2 us; 131,072 Q3 quadrilaterals 17, 12, 12 us.
 template <int DIM, int P>
 struct MC : TC<DIM, P> {
   using C = TC<DIM, P>;
-  static constexpr int EB = C::ND <= 4 ? 128 : (C::ND <= 9 ? 64 : (C::ND <= 27 ? 32 : 16));
+  static constexpr int S = DIM == 3 ? (P == 1 ? 1 : 1 << P) : (P <= 2 ? 1 : (P == 3 ? 2 : 4));
+  static constexpr int EB = 64 / S;
+  static constexpr int BLOCK = 64 * C::NEQ;
+  static constexpr int A = 4;
   static constexpr int NDP = C::ND | 1;  // odd row length: the summing lanes hit different LDS banks
 };
 template <int DIM, int P>
-__global__ __launch_bounds__(256) void tensor_means_kernel(const MeansArgs A,
-                                                           const TensorTables* __restrict__ gtb) {
+__global__ __launch_bounds__(64 * (DIM + 2)) void tensor_means_kernel(const MeansArgs args,
+                                                                      const TensorTables* __restrict__ gtb) {
   using C = MC<DIM, P>;
-  constexpr int N = C::N, ND = C::ND, NEQ = C::NEQ, EB = C::EB, NDP = C::NDP;
+  constexpr int N = C::N, ND = C::ND, NEQ = C::NEQ, EB = C::EB, NDP = C::NDP, S = C::S, A = C::A;
   __shared__ double s_u[NEQ][EB][NDP];
   __shared__ double s_w[DIM == 3 ? EB : 1][NDP];  // curved elements: each its own weights
   const int tid = threadIdx.x;
-  const int64_t NE = A.NE, NDOFS = NE * ND;
+  const int64_t NE = args.NE, NDOFS = NE * ND;
   const int64_t e0 = (int64_t)blockIdx.x * EB;
   const int ne = NE - e0 < EB ? (int)(NE - e0) : EB;
-  const bool curved = DIM == 3 && A.cgeo != nullptr;
-  constexpr int LP = (EB * ND + 255) / 256;
+  const bool curved = DIM == 3 && args.cgeo != nullptr;
+  constexpr int LP = (EB * ND + C::BLOCK - 1) / C::BLOCK;
 #pragma unroll
   for (int p = 0; p < LP; p++) {
-    const int i = tid + 256 * p;
+    const int i = tid + C::BLOCK * p;
     if (i < ne * ND) {
       const int el = i / ND, k = i - el * ND;
 #pragma unroll
-      for (int v = 0; v < NEQ; v++) s_u[v][el][k] = A.x[v * NDOFS + e0 * ND + i];
-      if (curved) s_w[DIM == 3 ? el : 0][k] = A.cgeo[(e0 + el) * CurvedLayout<P>::size + CurvedLayout<P>::mw + k];
+      for (int v = 0; v < NEQ; v++) s_u[v][el][k] = args.x[v * NDOFS + e0 * ND + i];
+      if (curved) s_w[DIM == 3 ? el : 0][k] = args.cgeo[(e0 + el) * CurvedLayout<P>::size + CurvedLayout<P>::mw + k];
     }
   }
   if (!curved && tid < ND) {
@@ -846,19 +851,33 @@ __global__ __launch_bounds__(256) void tensor_means_kernel(const MeansArgs A,
     s_w[0][tid] = w;
   }
   __syncthreads();
-  for (int i = tid; i < EB * NEQ; i += 256) {
-    const int v = i / EB, el = i - v * EB;
-    if (el < ne) {
-      const double* w = s_w[curved ? el : 0];
-      double s = 0.0, ws = 0.0;
+  const int v = tid / 64, el = tid % 64 / S, part = tid % S;
+  const double* u = s_u[v][el < ne ? el : 0];
+  const double* w = s_w[curved && el < ne ? el : 0];
+  double s[A], ws[A];
 #pragma unroll
-      for (int k = 0; k < ND; k++) {
-        s += w[k] * s_u[v][el][k];
-        ws += w[k];
-      }
-      A.means[v * NE + e0 + el] = s / ws;
+  for (int j = 0; j < A; j++) s[j] = ws[j] = 0.0;
+#pragma unroll
+  for (int t = 0; t * S < ND; t++) {
+    const int k = part + S * t;
+    if (k < ND) {
+      s[t % A] += w[k] * u[k];
+      ws[t % A] += w[k];
     }
   }
+#pragma unroll
+  for (int h = A / 2; h > 0; h /= 2)
+#pragma unroll
+    for (int j = 0; j < h; j++) {
+      s[j] += s[j + h];
+      ws[j] += ws[j + h];
+    }
+#pragma unroll
+  for (int off = S / 2; off > 0; off /= 2) {
+    s[0] += __shfl_xor(s[0], off, 64);
+    ws[0] += __shfl_xor(ws[0], off, 64);
+  }
+  if (el < ne && part == 0) args.means[v * NE + e0 + el] = s[0] / ws[0];
 }
 
 // ---------------------------------------------------------------------------
@@ -1356,7 +1375,7 @@ hipError_t launch_tensor_means(int dim, int p, const MeansArgs& a, const TensorT
 #define X(D, PP)                                                                      \
   if (dim == D && p == PP) {                                                          \
     using C = MC<D, PP>;                                                              \
-    tensor_means_kernel<D, PP><<<(unsigned)((a.NE + C::EB - 1) / C::EB), 256, 0, s>>>(a, t); \
+    tensor_means_kernel<D, PP><<<(unsigned)((a.NE + C::EB - 1) / C::EB), C::BLOCK, 0, s>>>(a, t); \
     return hipGetLastError();                                                         \
   }
   RKDG_TENSOR_CASES(X)

@@ -909,6 +909,15 @@ struct LC : TC<DIM, P> {
   static constexpr int ROW = C::ND + (C::ND & 1);
   static constexpr int want = DIM == 3 ? 4 : 2;
   static constexpr int ES = C::NEQ * ROW + (32 + want - (C::NEQ * ROW) % 32) % 32;
+  // A mesh with at most one workgroup per CU (256) waits for the chain of one lane:
+  // there, from the orders whose chain is long enough to matter, a workgroup takes a
+  // wavefront per variable, the first for the indicator and the others each for
+  // their variable at the vertices (729 Q3 hexahedra 8.7 -> 5.0 us, a team of 64
+  // lanes per element took 6.7; 440 Q2 6.8 -> 5.2, 5.9; 900 Q5 quadrilaterals 6.8
+  // -> 4.8, 5.8). With more workgroups it loses (2360 Q2 hexahedra 7.0 -> 8.2 us;
+  // 32,768 14 -> 52 us): their wavefronts fill the chip by themselves.
+  static constexpr bool WIDE = DIM == 3 ? P >= 2 : P >= 4;
+  static constexpr int64_t WIDE_BLOCKS = 256;
 };
 
 template <int ctrl>
@@ -937,10 +946,11 @@ __device__ __forceinline__ double team_max(double x) {
   return -team_min<T>(-x);
 }
 
-template <int DIM, int P>
-__global__ __launch_bounds__(64, 2) void tensor_limit_kernel(const LimitArgs A, const SchemeParams g,
-                                                          const TensorTables* __restrict__ gtb) {
+template <int DIM, int P, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void tensor_limit_kernel(const LimitArgs A, const SchemeParams g,
+                                                               const TensorTables* __restrict__ gtb) {
   using C = LC<DIM, P>;
+  static_assert(NW == 1 || (NW == C::NEQ && P > 1), "one wavefront, or one per variable");
   constexpr int N = C::N, ND = C::ND, NEQ = C::NEQ, NF = C::NF, T = C::T, EPB = C::EPB;
   constexpr int ROW = C::ROW, ES = C::ES;
   constexpr int NZ = DIM == 3 ? N : 1;
@@ -948,8 +958,10 @@ __global__ __launch_bounds__(64, 2) void tensor_limit_kernel(const LimitArgs A, 
   __shared__ double s_tab[4 * N];                                // E[2][N], BI[2][N]
   __shared__ double s_mean[EPB][NEQ];
   __shared__ double s_f[EPB];
+  __shared__ double s_v[NW > 1 ? NW : 1][64];  // the variables at the vertices, one wavefront each
 
-  const int tid = threadIdx.x;
+  const int tid = NW > 1 ? threadIdx.x % 64 : threadIdx.x;
+  const int wave = NW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / 64) : 0;
   const int team = tid / T, lane = tid % T;
   const int64_t NE = A.NE;
   const int64_t NDOFS = NE * ND;
@@ -957,30 +969,30 @@ __global__ __launch_bounds__(64, 2) void tensor_limit_kernel(const LimitArgs A, 
   const int64_t e = e0 + team;
   const bool active = e < NE;
   if (g.limiter == RKDG_LIM_NONE) {
-    if (A.troubled && active && lane == 0) A.troubled[e] = 0;
-    if (A.factor && active && lane == 0) A.factor[e] = 1.0;
+    if (A.troubled && active && wave == 0 && lane == 0) A.troubled[e] = 0;
+    if (A.factor && active && wave == 0 && lane == 0) A.factor[e] = 1.0;
     return;
   }
   const bool multi = g.limiter == RKDG_LIM_MULTI, findiff = g.limiter == RKDG_LIM_FINDIFF;
   const int vsel = findiff ? NEQ - 1 : 0;
 
   // every load of the setup is issued before the first LDS store
-  constexpr int LP = (EPB * ND + 63) / 64;
+  constexpr int LP = (EPB * ND + 64 * NW - 1) / (64 * NW);
   const int nn = (int)((NE - e0 < EPB ? NE - e0 : EPB) * ND);  // nodes of this block's elements
   double st[LP][NEQ];
 #pragma unroll
   for (int p = 0; p < LP; p++) {
-    const int i = tid + 64 * p;
+    const int i = threadIdx.x + 64 * NW * p;
 #pragma unroll
     for (int v = 0; v < NEQ; v++) st[p][v] = i < nn ? sbase(A.x + (v * NDOFS + e0 * ND))[(unsigned)i] : 1.0;
   }
-  const double tabv = tid < 4 * N ? (tid < 2 * N ? gtb->E[tid / N][tid % N] : gtb->BI[tid / N - 2][tid % N]) : 0.0;
+  const double tabv = wave == 0 && tid < 4 * N ? (tid < 2 * N ? gtb->E[tid / N][tid % N] : gtb->BI[tid / N - 2][tid % N]) : 0.0;
   // the element's means (lane v < NEQ) and the deciding variable's means of the
   // face neighbours (lane lf < NF): one load instruction each
   static_assert(NEQ <= T && NF <= T, "one lane per variable and per face");
   const bool ind_bj = g.indicator == RKDG_IND_BJ;
-  const double mown = (active && lane < NEQ) ? A.means[lane * NE + e] : 0.0;
-  const int nbl = (active && ind_bj && lane < NF) ? A.nbr[lane * NE + e] : -1;
+  const double mown = (active && wave == 0 && lane < NEQ) ? A.means[lane * NE + e] : 0.0;
+  const int nbl = (active && ind_bj && wave == 0 && lane < NF) ? A.nbr[lane * NE + e] : -1;
   // a neighbour whose mean is not a number bounds nothing (team_min would carry it
   // to some of the lanes)
   const double nm = nbl >= 0 ? A.means[vsel * NE + nbl] : NAN;
@@ -1009,17 +1021,17 @@ __global__ __launch_bounds__(64, 2) void tensor_limit_kernel(const LimitArgs A, 
     const double k3 = g.venkat_k * g.venkat_k * g.venkat_k;
     eps2 = k3 * (DIM == 3 ? dj : dj * sqrt(dj));
   }
-  if (tid < 4 * N) s_tab[tid] = tabv;
+  if (wave == 0 && tid < 4 * N) s_tab[tid] = tabv;
 #pragma unroll
   for (int p = 0; p < LP; p++) {
-    const int i = tid + 64 * p;
+    const int i = threadIdx.x + 64 * NW * p;
     if (i < EPB * ND) {
       const int el = i / ND, k = i - el * ND;
 #pragma unroll
       for (int v = 0; v < NEQ; v++) s_u[el * ES + v * ROW + k] = st[p][v];
     }
   }
-  if (lane < NEQ) s_mean[team][lane] = mown;
+  if (wave == 0 && lane < NEQ) s_mean[team][lane] = mown;
   __syncthreads();
   double mean[NEQ];
 #pragma unroll
@@ -1064,7 +1076,9 @@ __global__ __launch_bounds__(64, 2) void tensor_limit_kernel(const LimitArgs A, 
   };
   double vs[NEQ];  // the state at the vertex
   double yr = 1e9;
-  if (ind_bj) {
+  if (wave > 0) {
+    if (multi && g.last_hope) s_v[NW > 1 ? wave : 0][tid] = at_vertex(ue + wave * ROW);
+  } else if (ind_bj) {
     // the deciding variable at the vertex and at the lane's point on the face
     // normal to each axis
     double pt[DIM], V = 0.0;
@@ -1125,6 +1139,7 @@ __global__ __launch_bounds__(64, 2) void tensor_limit_kernel(const LimitArgs A, 
     }
     yr = team_min<T>(yr);
   }
+  if (NW > 1) __syncthreads();
   if (g.indicator == RKDG_IND_NOWHERE) yr = 1.0;
   else if (g.indicator == RKDG_IND_EVERYWHERE) yr = 0.0;
 
@@ -1145,7 +1160,7 @@ __global__ __launch_bounds__(64, 2) void tensor_limit_kernel(const LimitArgs A, 
 
   int trouble = 0;
   double f = 1.0;  // the factor of the limited state mean + f (u - mean)
-  if (multi) {
+  if (multi && wave == 0) {
     if (yr < 1.0) trouble = 1;
     // u <- mean + y (u - mean) applied nd times (limiter_multiplier.cpp:24-38)
     // is u <- mean + y^nd (u - mean); y^nd by repeated squaring
@@ -1163,7 +1178,8 @@ __global__ __launch_bounds__(64, 2) void tensor_limit_kernel(const LimitArgs A, 
       // the limited state at the reference vertices: mean + f (u(vertex) - mean)
 #pragma unroll
       for (int v = 0; v < NEQ; v++) {
-        if (v > 0 || !ind_bj || linear) vs[v] = at_vertex(ue + v * ROW);
+        if (NW > 1 && v > 0) vs[v] = s_v[v][tid];
+        else if (v > 0 || !ind_bj || linear) vs[v] = at_vertex(ue + v * ROW);
         vs[v] = mean[v] + f * (vs[v] - mean[v]);
       }
       const unsigned long long bm = __ballot(!physical<DIM>(vs, g));
@@ -1172,22 +1188,22 @@ __global__ __launch_bounds__(64, 2) void tensor_limit_kernel(const LimitArgs A, 
         f = 0.0;
       }
     }
-  } else if (findiff) {
+  } else if (findiff && wave == 0) {
     if (yr < 0.999) {
       trouble = 1;
       f = 0.0;
     }
   }
-  if (A.troubled && active && lane == 0) A.troubled[e] = (int8_t)trouble;
+  if (A.troubled && active && wave == 0 && lane == 0) A.troubled[e] = (int8_t)trouble;
   if (A.factor) {
-    if (active && lane == 0) A.factor[e] = f;
+    if (active && wave == 0 && lane == 0) A.factor[e] = f;
     return;
   }
-  if (lane == 0) s_f[team] = f;
+  if (wave == 0 && lane == 0) s_f[team] = f;
   __syncthreads();
 #pragma unroll
   for (int p = 0; p < LP; p++) {
-    const int i = tid + 64 * p;
+    const int i = threadIdx.x + 64 * NW * p;
     if (i < nn) {
       const int el = i / ND, k = i - el * ND;
       const double fe = s_f[el];
@@ -1362,7 +1378,10 @@ hipError_t launch_tensor_limit(int dim, int p, const LimitArgs& a, const SchemeP
   if (dim == D && p == PP) {                                               \
     using C = LC<D, PP>;                                                   \
     const int64_t nb = (a.NE + C::EPB - 1) / C::EPB;                       \
-    tensor_limit_kernel<D, PP><<<(unsigned)nb, 64, 0, s>>>(a, g, t);       \
+    if (C::WIDE && nb <= C::WIDE_BLOCKS)                                   \
+      tensor_limit_kernel<D, PP, C::WIDE ? C::NEQ : 1><<<(unsigned)nb, 64 * C::NEQ, 0, s>>>(a, g, t); \
+    else                                                                   \
+      tensor_limit_kernel<D, PP, 1><<<(unsigned)nb, 64, 0, s>>>(a, g, t);  \
     return hipGetLastError();                                              \
   }
   RKDG_TENSOR_CASES(X)

@@ -993,11 +993,8 @@ __global__ __launch_bounds__(64 * NW, 2) void tensor_limit_kernel(const LimitArg
   const bool ind_bj = g.indicator == RKDG_IND_BJ;
   const double mown = (active && wave == 0 && lane < NEQ) ? A.means[lane * NE + e] : 0.0;
   const int nbl = (active && ind_bj && wave == 0 && lane < NF) ? A.nbr[lane * NE + e] : -1;
-  // a neighbour whose mean is not a number bounds nothing (team_min would carry it
-  // to some of the lanes)
-  const double nm = nbl >= 0 ? A.means[vsel * NE + nbl] : NAN;
-  double nml = nm == nm ? nm : 1e300;
-  double nmh = nm == nm ? nm : -1e300;
+  double nml = nbl >= 0 ? A.means[vsel * NE + nbl] : 1e300;
+  double nmh = nbl >= 0 ? nml : -1e300;
   bool has_nb = nbl >= 0;
   if (A.ncnb && nbl <= kNcCode0) {  // a non-conforming face: the bounds over its neighbours
     const int k = kNcCode0 - nbl;
@@ -1040,8 +1037,10 @@ __global__ __launch_bounds__(64 * NW, 2) void tensor_limit_kernel(const LimitArg
   double msel = findiff ? mean[NEQ - 1] : mean[0];
   double mI = 1e9, MI = -1e9;
   if (ind_bj) {
-    mI = team_min<T>(nml);
-    MI = team_max<T>(nmh);
+    // a neighbour whose mean is not a number bounds nothing (team_min would carry it
+    // to some of the lanes); looked at here, where the means have arrived
+    mI = team_min<T>(nml == nml ? nml : 1e300);
+    MI = team_max<T>(nmh == nmh ? nmh : -1e300);
     mI = mI < msel ? mI : msel;
     MI = MI > msel ? MI : msel;
   }

@@ -119,7 +119,7 @@ def measured_traffic(n):
 # ADD) per wave from the SQ_INSTS_VALU_{FMA,MUL,ADD}_F64 counters of the plain
 # RHS at 96^3, two elements per wave (idle lanes included: an upper bound on
 # useful FLOPs; the stage epilogue's few axpy FLOPs per DOF are left out)
-RHS_FLOP_PER_ELEMENT = 45952
+RHS_FLOP_PER_ELEMENT = 45344
 FP64_PEAK_TFLOPS = 78.6
 
 

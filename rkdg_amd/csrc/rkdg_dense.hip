@@ -31,7 +31,9 @@ namespace rkdg {
 // element reads 2 NF doubles of its record, and the inverse mass is folded into
 // the volume and lift tables (triangles) or diagonal (quadrilaterals).
 //
-// Bound by FP64 issue and latency at 3 to 5 waves per SIMD. Limited steps, at
+// Bound by VALU issue (Q1 quadrilaterals: 69 % busy, LDS 47 %) or latency (P2
+// triangles 45 % and 53 %) at four waves per SIMD, three at order 3 and five for P1
+// triangles: the LDS of a wave (8.9 to 15.5 KB) sets it. Limited steps, at
 // first (power-of-two teams, every point reading the whole neighbour, dense
 // inverse mass and a full geometry record per element, the persistent loop) and
 // now, with the limiter's own change: 27,467 bilinear Q2 quadrilaterals, two
@@ -81,8 +83,8 @@ __device__ __forceinline__ void dense_rhs_block(const RhsArgs& A, const SchemePa
   __shared__ double s_nrm[EPB][2 * NF];
   __shared__ int s_nb[EPB][NF], s_code[EPB][NF];
 
-  // opaque to the compiler, so that the LDS addresses formed from it are not
-  // kept over the persistent loop (they held 160 registers and spilled)
+  // opaque to the compiler, so that the persistent form (LOOP) does not keep the LDS
+  // addresses formed from it over its loop (they held 160 registers and spilled)
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));
   const int team = tid / T, lane = tid - team * T;

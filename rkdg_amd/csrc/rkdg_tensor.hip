@@ -17,8 +17,8 @@
 // points, Riemann solve, lift back. Every face flux is evaluated with the
 // arguments ordered as (Elem1 state, Elem2 state, Elem1 normal), or, for the
 // Rusanov flux on hexahedra, which has the symmetry bit by bit, with the own
-// side first and the outward normal: both elements of a face see bitwise
-// identical fluxes and the scheme is conservative to round-off. Kernels are specialised on the Riemann solver and
+// side first and the outward normal: from the same traces both elements of a face
+// form bitwise identical fluxes, and the scheme is conservative to round-off. Kernels are specialised on the Riemann solver and
 // on the presence of boundary faces.
 #include <cstring>
 
@@ -196,7 +196,8 @@ __global__ __launch_bounds__(64, (ROLE == 1 ? 4 : rhs_waves<DIM, P, RS, BC, CV>(
   // still see the same bits; the rotated solvers need the canonical order. It
   // takes ten selects out of every face point (3032 Q2 hexahedra with hanging
   // nodes: step 150 -> 142 us; the 96^3 step is bound by LDS and stays as it was).
-  // At order 3 it costs spills (Q3: 119 VGPRs and none -> 128 and 4 to 6)
+  // At order 3 it cost spills while the compiler chose what to contract (Q3: 119
+  // VGPRs and none -> 128 and 4 to 6)
   constexpr bool OUTWARD = RS == RKDG_RS_RUSANOV && DIM == 3 && P <= 2;
   constexpr int ES = SOLVE ? EPB : 1;  // extent of the arrays only the face solves use
   constexpr int FB = NF * NEQ * NFN;   // lifted face fluxes of one receiver element

@@ -710,6 +710,12 @@ __global__ __launch_bounds__(64, 4) void dense_limit_kernel(const LimitArgs A, c
         f = 0.0;
       }
     }
+    // an element with a mean that is not finite is written also where the factor is 1:
+    // mean + f (u - mean) leaves no node of that variable finite
+    double t = 0.0;
+#pragma unroll
+    for (int v = 0; v < NEQ; v++) t += 0.0 * mean[v];
+    if (f == 1.0 && !(t == 0.0)) f = 0x1.fffffffffffffp-1;
   } else if (findiff) {
     if (yr < 0.999) {
       trouble = 1;

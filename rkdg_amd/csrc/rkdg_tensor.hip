@@ -1188,6 +1188,12 @@ __global__ __launch_bounds__(64 * NW, 2) void tensor_limit_kernel(const LimitArg
         f = 0.0;
       }
     }
+    // an element with a mean that is not finite is written also where the factor is 1:
+    // mean + f (u - mean) leaves no node of that variable finite
+    double t = 0.0;
+#pragma unroll
+    for (int v = 0; v < NEQ; v++) t += 0.0 * mean[v];
+    if (f == 1.0 && !(t == 0.0)) f = 0x1.fffffffffffffp-1;
   } else if (findiff && wave == 0) {
     if (yr < 0.999) {
       trouble = 1;
